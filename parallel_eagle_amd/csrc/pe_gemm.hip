@@ -42,6 +42,7 @@
 #include "pe_common.h"
 #include "pe_internal.h"
 
+#include <cmath>
 #include <cstdlib>
 #include <type_traits>
 
@@ -1094,119 +1095,243 @@ __global__ __launch_bounds__(kWaves * 64, 2) void dense_gemm_bigm_kernel(const u
 // ---------------------------------------------------------------------------
 // Dense 16-bit GEMM over many rows: 256 x 256 output tiles
 // ---------------------------------------------------------------------------
-// One workgroup = 4 waves = 256 rows (eight 32-row tiles of the A-tiled X) x
-// 256 columns (eight 32-column weight tiles); wave w owns rows 128 (w / 2) ..
-// + 127 and columns 128 (w % 2) .. + 127: 4 x 4 MFMA tiles, 256 fp32
-// accumulators. K is walked in stages of two MFMA k-steps. A stage's 16 A
-// fragments (8 M tiles x 2 k-steps) and 16 B fragments (8 N tiles x 2
-// k-steps), 1 KiB each, go straight from global memory into a four-stage LDS
-// ring (global_load_lds_dwordx4: three stages in flight while one is
-// multiplied); wave w loads fragments 8 w .. 8 w + 7 of the stage (A for
-// w < 2, B otherwise). A fragments are copied as stored (the A-tiled layout is
-// MFMA fragment order). The B fragment for k-step s of unit p is gathered lane
-// by lane from weight k-step 8 p + 4 g + s / 2, lane n + 32 (s % 2) of the
-// tiled weights, so that both operands hold the same k in the same place. Per
-// stage a wave reads its 4 + 4 fragments of each k-step (ds_read_b128 at the
-// lane's 16 bytes: conflict-free) and issues 32 MFMAs. One vmcnt wait and one
-// barrier per stage; loads past the split's last stage repeat its last unit
-// into buffers nobody reads. Work item w of the grid (column tile w / mblocks,
-// row block w % mblocks) runs on XCD w / (grid / 8) when the grid is a
-// multiple of eight, so the row blocks of a column tile share its weights in
-// one L2. grid.y: K splits (fp32 partials out[split][row][col]).
-constexpr int kT256Stage = 32 * 1024;
-constexpr int kT256Ring = 4;
-// s_waitcnt with vmcnt = 16 (expcnt and lgkmcnt at their maxima): this wave's
-// loads of the two later stages in flight may still be outstanding
-constexpr int kWaitVm16 = (16 & 15) | (7 << 4) | (15 << 8) | ((16 >> 4) << 14);
+// One workgroup = 4 waves = a block of up to 256 rows (32-row tiles of the
+// A-tiled X) x 256 columns (eight 32-column weight tiles); wave w owns the
+// row tiles MI (w / 2) .. + MI - 1 and the columns 128 (w % 2) .. + 127: MI x 4
+// MFMA tiles (MI = 4: 256 fp32 accumulators). The last row block of a launch
+// runs MI = 2 or 1 when it holds at most four or two tiles (777 rows: 3 x 256
+// + 9, the 9 rows at the price of 64).
+//
+// K is walked in stages of two MFMA k-steps. A stage's 4 MI A fragments and 16
+// B fragments, 1 KiB each, go straight from global memory into an LDS ring of
+// R stages (global_load_lds_dwordx4), R - 1 stages ahead; the four waves load
+// MI + 4 fragments each. A fragments are copied as stored (the A-tiled layout
+// is MFMA fragment order). The B fragment for k-step s of unit p is gathered
+// lane by lane from weight k-step 8 p + 4 g + s / 2, lane n + 32 (s % 2) of the
+// tiled weights, so that both operands hold the same k in the same place.
+//
+// One wave per SIMD, so a wave hides its own latencies: the fragments of the
+// next k-step are read into a second register set between the MFMAs of the
+// current one, the stage's one barrier sits in front of its second k-step
+// (whose operands are already in registers; behind it the next stage's first
+// fragments are read), and the loads of the ring are issued between the MFMAs
+// of the first k-step. A barrier at the stage's start, followed by the loads
+// and the reads of the fragments its MFMAs wait for, left the matrix cores idle
+// for half of every stage. Measured: 777 x 152064 x 5120 (fp16 lm_head) 1742 ->
+// 1190 us (1.02 PFLOP/s), 2000 x 22016 x 4096 417 -> 320 us; bound by the MFMA
+// issue of one wave per SIMD (0.5 us a stage with 64 workgroups, 0.8 us with
+// all CUs busy, where the clock falls), 5-10 us a tile for the ring's first
+// stages and the epilogue, and the last round of tiles.
+//
+// Epilogues: fp32 sums out[split][row][col] (EPI 1); 16-bit values (EPI 0) and
+// the SwiGLU activation stored A-tiled (EPI 2) with the operands' roles
+// swapped, so that a lane holds four consecutive columns of one row: the
+// 16-bit tile goes through the ring's LDS (16-byte chunk c of row m at
+// c ^ (m % 16)) to whole 256-byte row pieces, and a store of the A-tiled
+// activation covers 512 contiguous bytes.
+// Work item w of the grid (column tile w / mblocks, row block w % mblocks)
+// runs on XCD w / (grid / 8), so the row blocks of a column tile share its
+// weights in one L2. grid.y: K splits (EPI 1).
+constexpr int kEpiT16 = 0, kEpiTF32 = 1, kEpiTSwiglu = 2;
+constexpr int kT256Smem = 144 * 1024;
+constexpr int t256_stage(int MI) { return (4 * MI + 16) * 1024; }
+constexpr int t256_ring(int MI) { return kT256Smem / t256_stage(MI); }  // 4, 6 and 7 stages
+// s_waitcnt immediate: vmcnt = n, lgkmcnt = 0, expcnt at its maximum
+constexpr int wait_vm_lgkm0(int n) { return (n & 15) | (7 << 4) | ((n >> 4) << 14); }
 
-template <int DT, bool F32OUT>
-__global__ __launch_bounds__(256, 1) void dense_gemm_t256_kernel(const uint16_t* __restrict__ X,
-                                                                 const uint16_t* __restrict__ W, int units,
-                                                                 int ups, int mtiles, int mblocks, int M,
-                                                                 void* __restrict__ out, int64_t ld, int64_t N) {
-  __shared__ __align__(1024) uint8_t smem[kT256Ring * kT256Stage];
-  const int total = gridDim.x;
-  const int b = blockIdx.x;
-  const int w = (total & 7) ? b : (b & 7) * (total >> 3) + (b >> 3);
-  const int ntile = w / mblocks, mblock = w - ntile * mblocks;
-  const int split = blockIdx.y;
-  const int u0 = split * ups, u1 = min(units, u0 + ups);
-  if (u0 >= u1) return;
-  const int nstages = (u1 - u0) * 4;
+struct T256Args {
+  const uint16_t* x;
+  const uint16_t* w;
+  int units, ups;      // 128-wide K units: all, and per split
+  int mtiles, mblocks, bt; // 32-row tiles, and blocks of bt (8, 4 or 2) of them
+  int M;
+  void* out;
+  int64_t ld;     // row stride of out in elements (16-bit and fp32 outputs)
+  int out_units;  // SwiGLU: 128-column units of the A-tiled activation
+  int vec;        // 16-bit output: rows and base 16-byte aligned
+};
+
+template <int DT, int MI, int EPI>
+__device__ __forceinline__ void t256_tile(uint8_t* smem, const T256Args& p, int ntile, int mblock, int split, int u0,
+                                          int nst) {
+  constexpr int STG = t256_stage(MI), R = t256_ring(MI), PW = MI + 4, AF = 4 * MI;
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int ln = lane & 31, g = lane >> 5;
-  const int KS = units * 8;  // weight k-steps
   const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem;
-  const uint16_t* xb = uniform_ptr(X);
-  const uint16_t* wb = uniform_ptr(W);
-  // this wave's eight fragments of a stage
-  auto issue = [&](int t) {
-    const int tc = min(t, nstages - 1);
-    const int p = u0 + tc / 4, s0 = 2 * (tc % 4);
-    const uint32_t dst = __builtin_amdgcn_readfirstlane(lds_base + (t % kT256Ring) * kT256Stage + wave * 8192);
+  const uint8_t* xb = (const uint8_t*)uniform_ptr(p.x);
+  const uint8_t* wb = (const uint8_t*)uniform_ptr(p.w);
+  // byte offsets of this wave's fragments at unit 0; a stage adds a uniform amount
+  uint32_t voff[PW];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int f = 8 * (wave & 1) + i;  // fragment of the operand: tile f / 2, k-step s0 + f % 2
-      const int s = s0 + (f & 1);
-      uint32_t off;
-      if (wave < 2) {
-        const int mt = min(mblock * 8 + (f >> 1), mtiles - 1);
-        off = (uint32_t)((((mt * units + p) * 8 + s) * 64 + lane) * 16);
-      } else {
-        const int nt = ntile * 8 + (f >> 1);
-        off = (uint32_t)((((int64_t)nt * KS + 8 * p + 4 * g + (s >> 1)) * 64 + ln + 32 * (s & 1)) * 16);
-      }
-      lds_dma16(wave < 2 ? (const void*)xb : (const void*)wb, off, dst + i * 1024);
+  for (int i = 0; i < PW; ++i) {
+    const int f = wave * PW + i;
+    if (f < AF) {
+      const int mt = min(mblock * p.bt + (f >> 1), p.mtiles - 1);
+      voff[i] = (uint32_t)(((mt * p.units * 8 + (f & 1)) * 64 + lane) * 16);
+    } else {
+      const int nt = ntile * 8 + ((f - AF) >> 1);
+      voff[i] = (uint32_t)((((int64_t)nt * p.units * 8 + 4 * g) * 64 + ln + 32 * (f & 1)) * 16);
     }
-  };
-  const int wm = wave >> 1, wn = wave & 1;
-  f32x16_t acc[4][4];
+  }
+  // fragments i0 .. i1 - 1 of stage t (past the end: the last one again) into ring slot `slot`
+  auto issue = [&](int t, int slot, auto i0, auto i1) {
+    const int tt = u0 * 4 + min(t, nst - 1);
+    const uint8_t* xs = xb + (int64_t)tt * 2048;
+    const uint8_t* ws = wb + (int64_t)(8 * (tt >> 2) + (tt & 3)) * 1024;
+    const uint32_t dst = lds_base + slot * STG + wave * (PW * 1024);
 #pragma unroll
-  for (int mi = 0; mi < 4; ++mi)
+    for (int i = decltype(i0)::value; i < decltype(i1)::value; ++i)
+      lds_dma16(wave * PW + i < AF ? (const void*)xs : (const void*)ws, voff[i],
+                __builtin_amdgcn_readfirstlane(dst + i * 1024));
+  };
+  constexpr std::integral_constant<int, 0> kFirst{};
+  constexpr std::integral_constant<int, PW> kAll{};
+  const int wm = wave >> 1, wn = wave & 1;
+  f32x16_t acc[MI][4];
+#pragma unroll
+  for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
     for (int ni = 0; ni < 4; ++ni)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[mi][ni][r] = 0.f;
-  issue(0);
-  issue(1);
-  issue(2);
-  for (int t = 0; t < nstages; ++t) {
-    __builtin_amdgcn_s_waitcnt(kWaitVm16);  // this wave's loads of stage t have landed
-    __syncthreads();                        // everyone's have; stage t - 1's buffer is free
-    issue(t + 3);
-    const uint8_t* st = smem + (t % kT256Ring) * kT256Stage + lane * 16;
+  u32x4_t fa[2][MI], fb[2][4];
+  // fragment f (the four of B, then those of A) of k-step sl of the stage at `st`
+  auto read = [&](const uint8_t* st, int sl, int f) {
+    if (f < 4) fb[sl][f] = *(const u32x4_t*)(st + (AF + (4 * wn + f) * 2 + sl) * 1024 + lane * 16);
+    else fa[sl][f - 4] = *(const u32x4_t*)(st + ((MI * wm + f - 4) * 2 + sl) * 1024 + lane * 16);
+  };
+  auto mul = [&](int sl, int mi) {
 #pragma unroll
-    for (int sl = 0; sl < 2; ++sl) {
-      u32x4_t a[4], bf[4];
+    for (int ni = 0; ni < 4; ++ni)
+      acc[mi][ni] = EPI == kEpiTF32 ? mfma16<DT>(fa[sl][mi], fb[sl][ni], acc[mi][ni])
+                                    : mfma16<DT>(fb[sl][ni], fa[sl][mi], acc[mi][ni]);
+  };
 #pragma unroll
-      for (int mi = 0; mi < 4; ++mi) a[mi] = *(const u32x4_t*)(st + ((4 * wm + mi) * 2 + sl) * 1024);
+  for (int t = 0; t < R - 1; ++t) issue(t, t, kFirst, kAll);
+  __builtin_amdgcn_s_waitcnt(wait_vm_lgkm0((R - 2) * PW));
+  lds_barrier();
 #pragma unroll
-      for (int ni = 0; ni < 4; ++ni) bf[ni] = *(const u32x4_t*)(st + 16384 + ((4 * wn + ni) * 2 + sl) * 1024);
+  for (int f = 0; f < 4 + MI; ++f) read(smem, 0, f);
+  int slot = 0;  // of stage t
+  for (int t = 0; t < nst; ++t) {
+    const int next = slot + 1 == R ? 0 : slot + 1;
+    const int free_slot = slot == 0 ? R - 1 : slot - 1;  // stage t - 1's, read by nobody since the last barrier
+    const uint8_t* st = smem + slot * STG;
+    const uint8_t* sn = smem + next * STG;
+    // first k-step: the second one's fragments are read, stage t + R - 1 requested
 #pragma unroll
-      for (int mi = 0; mi < 4; ++mi)
+    for (int mi = 0; mi < MI; ++mi) {
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int ni = 0; ni < 4; ++ni) acc[mi][ni] = mfma16<DT>(a[mi], bf[ni], acc[mi][ni]);
+      for (int f = mi * (4 + MI) / MI; f < (mi + 1) * (4 + MI) / MI; ++f) read(st, 1, f);
+      if constexpr (MI == 4) {
+        if (mi == 0) issue(t + R - 1, free_slot, kFirst, std::integral_constant<int, 2>{});
+        if (mi == 1) issue(t + R - 1, free_slot, std::integral_constant<int, 2>{}, std::integral_constant<int, 4>{});
+        if (mi == 2) issue(t + R - 1, free_slot, std::integral_constant<int, 4>{}, std::integral_constant<int, 6>{});
+        if (mi == 3) issue(t + R - 1, free_slot, std::integral_constant<int, 6>{}, kAll);
+      } else if (mi == 0) {
+        issue(t + R - 1, free_slot, kFirst, kAll);
+      }
+      mul(0, mi);
     }
+    __builtin_amdgcn_sched_barrier(0);
+    // this wave has its last fragments of stage t, and its loads of stage t + 1 have landed
+    __builtin_amdgcn_s_waitcnt(wait_vm_lgkm0((R - 2) * PW));
+    lds_barrier();
+#pragma unroll
+    for (int mi = 0; mi < MI; ++mi) {
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int f = mi * (4 + MI) / MI; f < (mi + 1) * (4 + MI) / MI; ++f) read(sn, 0, f);
+      mul(1, mi);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    slot = next;
   }
-  __builtin_amdgcn_s_waitcnt(0);  // the ring's last loads land before the workgroup ends
-  typedef typename Elem<DT>::T Te;
-  const int64_t base = F32OUT ? (int64_t)split * M * ld : 0;
+  __builtin_amdgcn_s_waitcnt(0);  // the ring's last loads land before it is reused or the workgroup ends
+  const int row0 = mblock * p.bt * 32 + 32 * MI * wm, col0 = ntile * 256 + 128 * wn;
+  if constexpr (EPI == kEpiTF32) {
+    float* out = (float*)p.out + (int64_t)split * p.M * p.ld;
 #pragma unroll
-  for (int mi = 0; mi < 4; ++mi)
+    for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int row = mblock * 256 + 128 * wm + 32 * mi + 8 * (r >> 2) + 4 * g + (r & 3);
-      if (row >= M) continue;
+      for (int r = 0; r < 16; ++r) {
+        const int row = row0 + 32 * mi + 8 * (r >> 2) + 4 * g + (r & 3);
+        if (row >= p.M) continue;
 #pragma unroll
-      for (int ni = 0; ni < 4; ++ni) {
-        const int64_t o = base + (int64_t)row * ld + ntile * 256 + 128 * wn + 32 * ni + ln;
-        if constexpr (F32OUT)
-          ((float*)out)[o] = acc[mi][ni][r];
-        else
-          Elem<DT>::store((Te*)out, o, acc[mi][ni][r]);
+        for (int ni = 0; ni < 4; ++ni) out[(int64_t)row * p.ld + col0 + 32 * ni + ln] = acc[mi][ni][r];
+      }
+  } else if constexpr (EPI == kEpiTSwiglu) {
+    typedef Elem<DT> E;
+    // tiles 2 pr and 2 pr + 1 are the gate and up columns of 32 activation columns
+#pragma unroll
+    for (int mi = 0; mi < MI; ++mi) {
+      const int row = row0 + 32 * mi + ln;
+      if (row >= p.M) continue;
+#pragma unroll
+      for (int pr = 0; pr < 2; ++pr)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          float o[4];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const float gr = E::round(acc[mi][2 * pr][4 * q + j]), ur = E::round(acc[mi][2 * pr + 1][4 * q + j]);
+            o[j] = __fmul_rn(E::round(silu_f(gr)), ur);
+          }
+          const int col = (col0 >> 1) + 32 * pr + 8 * q + 4 * g;
+          Vec4<DT>::store((uint16_t*)p.out + xtile_index(row, col, p.out_units), o);
+        }
+    }
+  } else {
+    __syncthreads();  // every wave is done with the ring: it becomes the output tile
+    uint8_t* mine = smem + wave * (MI * 32 * 256);
+#pragma unroll
+    for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+      for (int ni = 0; ni < 4; ++ni)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int m = 32 * mi + ln, c = 4 * ni + q;
+          *(uint2*)(mine + m * 256 + ((c ^ (m & 15)) * 16) + 8 * g) =
+              make_uint2(pack2_16<DT>(acc[mi][ni][4 * q], acc[mi][ni][4 * q + 1]),
+                         pack2_16<DT>(acc[mi][ni][4 * q + 2], acc[mi][ni][4 * q + 3]));
+        }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+#pragma unroll 4
+    for (int it = 0; it < MI * 8; ++it) {
+      const int m = it * 4 + (lane >> 4), c = lane & 15;
+      const u32x4_t v = *(const u32x4_t*)(mine + m * 256 + ((c ^ (m & 15)) * 16));
+      if (row0 + m >= p.M) continue;
+      uint16_t* dst = (uint16_t*)p.out + (int64_t)(row0 + m) * p.ld + col0 + 8 * c;
+      if (p.vec) {
+        *(u32x4_t*)dst = v;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          dst[2 * e] = (uint16_t)v[e];
+          dst[2 * e + 1] = (uint16_t)(v[e] >> 16);
+        }
       }
     }
-  (void)N;
+  }
+}
+
+template <int DT, int EPI>
+__global__ __launch_bounds__(256, 1) void dense_gemm_t256_kernel(T256Args p) {
+  __shared__ __align__(1024) uint8_t smem[kT256Smem];
+  // XCD x runs a contiguous range of the work items
+  const int total = gridDim.x, b = blockIdx.x, x = b & 7;
+  const int w = x * (total >> 3) + min(x, total & 7) + (b >> 3);
+  const int ntile = w / p.mblocks, mblock = w - ntile * p.mblocks;
+  const int split = blockIdx.y;
+  const int u0 = split * p.ups, u1 = min(p.units, u0 + p.ups);
+  if (u0 >= u1) return;
+  const int left = min(p.bt, p.mtiles - mblock * p.bt);
+  if (left > 4) t256_tile<DT, 4, EPI>(smem, p, ntile, mblock, split, u0, (u1 - u0) * 4);
+  else if (left > 2) t256_tile<DT, 2, EPI>(smem, p, ntile, mblock, split, u0, (u1 - u0) * 4);
+  else t256_tile<DT, 1, EPI>(smem, p, ntile, mblock, split, u0, (u1 - u0) * 4);
 }
 
 // ---------------------------------------------------------------------------
@@ -1861,44 +1986,111 @@ int64_t pe_internal_nf4_bigm_partials_bytes(int M, int N, int K) {
   return (int64_t)big_plan(N, K).S * M * N * 4;
 }
 
+namespace {
+// Rows per workgroup (32 bt) and K splits of a t256 launch, by its estimated
+// time: rounds of one workgroup per CU, a workgroup taking kFixed + stages *
+// kStage[rows] (measured at N = 8192, K = 4096: 512 rows as 64, 128 and 256
+// workgroups of 256, 128 and 64 rows take 76, 55 and 41 us, 2048 rows as 256
+// full ones 110 us), and each split writing M x N fp32 sums that the consumer
+// reads again at about 4.5 TB/s.
+struct T256Plan {
+  int bt, S;
+};
+T256Plan t256_plan(int M, int N, int K, int max_splits, bool f32_out) {
+  constexpr double kFixed = 5.0;
+  auto stage_us = [](int tiles) { return tiles > 4 ? 0.80 : tiles > 2 ? 0.50 : 0.31; };
+  const int mt = (M + 31) / 32, units = K / 128, cu = cu_count();
+  T256Plan best = {8, 1};
+  double best_t = 1e30;
+  for (int bt = 8; bt >= 2; bt >>= 1) {
+    const int full = mt / bt, rem = mt % bt;
+    for (int S = 1; S <= max_splits && S <= units; ++S) {
+      const int ups = (units + S - 1) / S;
+      if ((units + ups - 1) / ups != S) continue;
+      const double cf = kFixed + 4 * ups * stage_us(bt), cr = kFixed + 4 * ups * stage_us(rem);
+      const double work = (double)(N / 256) * S * (full * cf + (rem ? cr : 0));
+      const double one = full ? cf : cr;
+      double t = std::ceil(work / (cu * one) - 1e-6) * one;
+      if (f32_out) t += (double)S * M * N * 8 / 4.5e6;
+      if (t < best_t) {
+        best_t = t;
+        best = {bt, S};
+      }
+    }
+  }
+  return best;
+}
+
+// Shapes of the t256 kernel: whole column tiles, byte offsets within X and W below 4 GiB.
+bool t256_shape(int M, int N, int K) {
+  return N % 256 == 0 && (int64_t)N * K * 2 < (int64_t(1) << 32) &&
+         (int64_t)((M + 31) / 32) * 32 * K * 2 < (int64_t(1) << 32);
+}
+
+int t256_launch(const void* x_tiled, int M, int K, const void* w, int dtype, int N, void* out, int64_t ld_out,
+                int epi, int out_units, T256Plan plan, hipStream_t st) {
+  T256Args a;
+  a.x = (const uint16_t*)x_tiled;
+  a.w = (const uint16_t*)w;
+  a.units = K / 128;
+  a.ups = (a.units + plan.S - 1) / plan.S;
+  a.mtiles = (M + 31) / 32;
+  a.bt = plan.bt;
+  a.mblocks = (a.mtiles + plan.bt - 1) / plan.bt;
+  a.M = M;
+  a.out = out;
+  a.ld = ld_out;
+  a.out_units = out_units;
+  a.vec = ((uintptr_t)out | (uintptr_t)(ld_out * 2)) % 16 == 0;
+  const dim3 grid((unsigned)(N / 256 * a.mblocks), plan.S);
+#define PE_T256(D)                                                                               \
+  do {                                                                                           \
+    if (epi == kEpiTF32) dense_gemm_t256_kernel<D, kEpiTF32><<<grid, 256, 0, st>>>(a);            \
+    else if (epi == kEpiTSwiglu) dense_gemm_t256_kernel<D, kEpiTSwiglu><<<grid, 256, 0, st>>>(a); \
+    else dense_gemm_t256_kernel<D, kEpiT16><<<grid, 256, 0, st>>>(a);                             \
+  } while (0)
+  if (dtype == PE_DTYPE_BF16) PE_T256(PE_DTYPE_BF16);
+  else if (dtype == PE_DTYPE_F16) PE_T256(PE_DTYPE_F16);
+  else return PE_ERR_ARG;
+#undef PE_T256
+  PE_CHECK_LAUNCH();
+  return PE_OK;
+}
+}  // namespace
+
+// The SwiGLU linear over many rows (N interleaved gate / up columns), the
+// activation stored A-tiled; PE_ERR_ARG for shapes without whole column tiles.
+bool pe_internal_dense_swiglu_fits(int M, int N, int K) { return K % 128 == 0 && t256_shape(M, N, K); }
+int pe_internal_dense_swiglu(const void* x_tiled, int M, int K, const void* w, int dtype, int N, void* act,
+                             int out_units, hipStream_t st) {
+  if (!x_tiled || !w || !act || M <= 0 || !pe_internal_dense_swiglu_fits(M, N, K) || out_units * 256 != N)
+    return PE_ERR_ARG;
+  return t256_launch(x_tiled, M, K, w, dtype, N, act, 0, kEpiTSwiglu, out_units, t256_plan(M, N, K, 1, false), st);
+}
+
+// splits: null, or receives the K splits of the fp32 partials, at most max_splits
 int pe_internal_dense_bigm(const void* x_tiled, int M, int K, const void* w, int dtype, int N, void* out,
-                           int64_t ld_out, hipStream_t st, bool f32_out, int* splits) {
+                           int64_t ld_out, hipStream_t st, bool f32_out, int* splits, int max_splits) {
   if (!x_tiled || !w || !out || M <= 0 || K % 128 || N % (32 * kBigNT) || ld_out < N) return PE_ERR_ARG;
   if (splits) *splits = 1;
-  const int mtiles0 = (M + 31) / 32;
-  // 256 x 256 tiles from an LDS ring when the tiles fill at least two rounds
-  // of one workgroup per CU (offsets within X and W below 4 GiB). With fewer
-  // tiles the 128-column kernel, two workgroups per CU, measured faster (a
-  // 2047-row drafter context: q/k/v 226 against 258 us, the 4096-column
-  // linears 212 against 285; gate/up, 688 tiles, 403 against 442)
-  const int mblocks0 = (M + 255) / 256;
-  if (M > 256 && N % 256 == 0 && (int64_t)(N / 256) * mblocks0 >= 512 && (int64_t)N * K * 2 < (int64_t(1) << 32) &&
-      (int64_t)mtiles0 * 32 * K * 2 < (int64_t(1) << 32)) {
-    const int units = K / 128, mblocks = mblocks0;
-    const dim3 grid((unsigned)(N / 256 * mblocks), 1);
-#define PE_T256_LAUNCH(D, F)                                                                                   \
-  dense_gemm_t256_kernel<D, F><<<grid, 256, 0, st>>>((const uint16_t*)x_tiled, (const uint16_t*)w, units, units, \
-                                                     mtiles0, mblocks, M, out, ld_out, N)
-    if (dtype == PE_DTYPE_BF16 && f32_out)
-      PE_T256_LAUNCH(PE_DTYPE_BF16, true);
-    else if (dtype == PE_DTYPE_BF16)
-      PE_T256_LAUNCH(PE_DTYPE_BF16, false);
-    else if (dtype == PE_DTYPE_F16 && f32_out)
-      PE_T256_LAUNCH(PE_DTYPE_F16, true);
-    else if (dtype == PE_DTYPE_F16)
-      PE_T256_LAUNCH(PE_DTYPE_F16, false);
-    else
-      return PE_ERR_ARG;
-#undef PE_T256_LAUNCH
-    PE_CHECK_LAUNCH();
-    return PE_OK;
+  // More than one row block: 256-column tiles from the LDS ring (M = 300, N =
+  // K = 4096: 39 against 72 us with the 128-column kernel; 1500 rows, K =
+  // 11008: 176 against 203; 777 rows of the 152064-column lm_head 1.2 against
+  // 1.7 ms). At most 256 rows of a wide lm_head are bound by its weights, read
+  // by twice as many workgroups in the 128-column kernel (208 rows: 433
+  // against 464 us).
+  if (M > 256 && t256_shape(M, N, K)) {
+    const T256Plan plan = t256_plan(M, N, K, splits && f32_out ? max_splits : 1, f32_out);
+    if (splits) *splits = plan.S;
+    return t256_launch(x_tiled, M, K, w, dtype, N, out, ld_out, f32_out ? kEpiTF32 : kEpiT16, 0, plan, st);
   }
   const int np = K / 128;
   const int mtiles = (M + 31) / 32;
   // fp32 partials for a caller that sums splits: two K splits when the column
   // groups x row blocks would fill fewer than two workgroups per CU
   int S = 1;
-  if (f32_out && splits && (int64_t)(N / (32 * kBigNT)) * ((mtiles + 7) / 8) < 512 && np >= 4) S = 2;
+  if (f32_out && splits && max_splits >= 2 && (int64_t)(N / (32 * kBigNT)) * ((mtiles + 7) / 8) < 512 && np >= 4)
+    S = 2;
   if (splits) *splits = S;
   const dim3 grid(N / (32 * kBigNT), (mtiles + 7) / 8, S);
 #define PE_DBIGM_LAUNCH(D, F)                                                                             \

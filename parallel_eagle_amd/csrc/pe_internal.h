@@ -53,19 +53,20 @@ PE_INTERNAL int pe_internal_rope_kv_partials(const float* partial, int S, int M,
                                              int64_t max_pos, void* q_out, void* k_cache, void* v_cache, int64_t cap,
                                              int64_t row0, int32_t* status, int dtype, hipStream_t st,
                                              const int64_t* kv_off = nullptr);
-// pe_gemm.hip: the NF4 GEMM for many rows (A-tiled X, 64 < M <= 256,
-// N % 128 == 0, fp16 absmax): each weight dequantised once for all rows;
-// fp32 split partials [S][M][N] (*splits receives S).
-// Dense 16-bit Y[M][N] = X . W^T for many rows (X A-tiled, W in the
-// MFMA-tiled layout, K % 128 == 0, N % 128 == 0), one workgroup per 128
-// columns and block of 256 rows, each weight read once per row block; Y
-// row-major (leading dimension ld_out) in the dtype, or the fp32 sums as they
-// are (f32_out: split partials [S][M][ld_out] for the prefill's epilogue
-// kernels; with `splits` given the launch may take S = 2 K splits and reports
-// S there, else S = 1).
+// pe_gemm.hip: 16-bit linear over many rows from A-tiled X (weights in the
+// MFMA-tiled layout, K % 128 == 0, N % 128 == 0), each weight read once per
+// block of up to 256 rows; Y row-major (leading dimension ld_out) in the
+// dtype, or the fp32 sums as they are (f32_out: split partials
+// [S][M][ld_out] for the prefill's epilogue kernels; with `splits` given the
+// launch takes up to max_splits K splits and reports S there, else S = 1).
 PE_INTERNAL int pe_internal_dense_bigm(const void* x_tiled, int M, int K, const void* w, int dtype, int N, void* out,
                                        int64_t ld_out, hipStream_t st, bool f32_out = false,
-                                       int* splits = nullptr);
+                                       int* splits = nullptr, int max_splits = 1);
+// The dense gate/up linear over many rows (N = 256 * out_units interleaved
+// columns) storing the SwiGLU activation A-tiled; shapes that fit only.
+PE_INTERNAL bool pe_internal_dense_swiglu_fits(int M, int N, int K);
+PE_INTERNAL int pe_internal_dense_swiglu(const void* x_tiled, int M, int K, const void* w, int dtype, int N, void* act,
+                                         int out_units, hipStream_t st);
 // The prefill's NF4 linear over all M rows (A-tiled X, blocks of 256 rows, one
 // K split): fp32 sums y[M][N], or with out_units > 0 (the interleaved gate/up
 // weight, N = 2 * 128 * out_units) the SwiGLU activation stored A-tiled.

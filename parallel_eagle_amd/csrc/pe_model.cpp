@@ -189,7 +189,7 @@ bool prefill_path(const pe_model_desc* m, int M, int mask_mode) {
 }
 
 struct PrefillLayout {
-  int64_t h, xn, xn_t, q, attn, attn_t, act_t, y, wdeq, wtile, attn_ws, attn_ws_bytes, gemm, gemm_bytes, total;
+  int64_t h, xn, xn_t, q, attn, attn_t, act_t, y, ny, wdeq, wtile, attn_ws, attn_ws_bytes, gemm, gemm_bytes, total;
 };
 
 PrefillLayout make_prefill_layout(const pe_model_desc* m, int M, int64_t kv_len) {
@@ -217,7 +217,8 @@ PrefillLayout make_prefill_layout(const pe_model_desc* m, int M, int64_t kv_len)
   int64_t ny = nqkv;
   if (2 * ip > ny) ny = 2 * ip;
   if (H > ny) ny = H;
-  L.y = take(M * ny * 4 * 2);  // up to two K splits of fp32 partials
+  L.ny = 2 * ny;  // fp32 partials: up to four K splits of the narrower linears, two of the widest
+  L.y = take(M * L.ny * 4);
   L.wdeq = L.wtile = 0;
   if (m->weight_format == PE_WFMT_NF4_F32ABS) {  // one linear dequantised, then tiled
     int64_t nw = nqkv * H;
@@ -291,20 +292,25 @@ int forward_prefill(const pe_model_desc* m, const pe_pass_args* a, const Prefill
     }
     return PE_OK;
   };
+  // a dense weight as stored, or fp32-absmax NF4 codes dequantised and tiled to 16 bits
+  auto dense_weight = [&](const void* w, const void* ab, int N, int K, const void** wt) -> int {
+    *wt = w;
+    if (m->weight_format != PE_WFMT_NF4_F32ABS) return PE_OK;
+    int r = pe_nf4_dequant_f32abs((const uint8_t*)w, (const float*)ab, N, K, (uint16_t*)(ws + Lp.wdeq), st);
+    if (r != PE_OK) return r;
+    *wt = ws + Lp.wtile;
+    return pe_dense_repack(ws + Lp.wdeq, N, K, m->dtype, ws + Lp.wtile, st);
+  };
   // y[ys][M][N] (fp32 split partials) = x (A-tiled) . W^T over all rows
   int ys = 1;
   auto linear = [&](const void* xt, int K, const void* w, const void* ab, int N) -> int {
     ys = 1;
     if (nf4) return pe_internal_nf4_prefill(xt, M, K, w, ab, N, y, nullptr, 0, st);
-    const void* wt = w;
-    if (m->weight_format == PE_WFMT_NF4_F32ABS) {
-      int r = pe_nf4_dequant_f32abs((const uint8_t*)w, (const float*)ab, N, K, (uint16_t*)(ws + Lp.wdeq), st);
-      if (r != PE_OK) return r;
-      r = pe_dense_repack(ws + Lp.wdeq, N, K, m->dtype, ws + Lp.wtile, st);
-      if (r != PE_OK) return r;
-      wt = ws + Lp.wtile;
-    }
-    return pe_internal_dense_bigm(xt, M, K, wt, m->dtype, N, y, N, st, true, &ys);
+    const void* wt;
+    const int r = dense_weight(w, ab, N, K, &wt);
+    if (r != PE_OK) return r;
+    const int most = (int)std::min<int64_t>(4, Lp.ny / N);
+    return pe_internal_dense_bigm(xt, M, K, wt, m->dtype, N, y, N, st, true, &ys, most);
   };
 
   {
@@ -332,6 +338,10 @@ int forward_prefill(const pe_model_desc* m, const pe_pass_args* a, const Prefill
                                         nullptr, 0, nullptr, 0, st));
     if (nf4) {
       PE_TRY(pe_internal_nf4_prefill(xn_t, M, H, m->w_gu[l], m->a_gu[l], 2 * ip, nullptr, act_t, ip / 128, st));
+    } else if (pe_internal_dense_swiglu_fits(M, 2 * ip, H)) {
+      const void* wt;
+      PE_TRY(dense_weight(m->w_gu[l], m->a_gu ? m->a_gu[l] : nullptr, 2 * ip, H, &wt));
+      PE_TRY(pe_internal_dense_swiglu(xn_t, M, H, wt, m->dtype, 2 * ip, act_t, ip / 128, st));
     } else {
       PE_TRY(linear(xn_t, H, m->w_gu[l], m->a_gu ? m->a_gu[l] : nullptr, 2 * ip));
       PE_TRY(pe_internal_swiglu_partials(y, ys, M, 2 * ip, act_t, ip, ip / 128, m->dtype, st));
