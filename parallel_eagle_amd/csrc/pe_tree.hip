@@ -120,47 +120,146 @@ __global__ __launch_bounds__(256) void bias_to_bits_kernel(const typename Elem<D
 // every number, and among equal maxima (or NaNs) the lowest index wins.
 constexpr int kArgThreads = 1024;
 
-// One block of kArgThreads per row. Thread t scans 16-byte vectors t,
-// t + kArgThreads, ... in increasing index order (all loads issued first)
-// keeping the first element of the largest key; the block then reduces with
-// (key descending, index ascending).
+// The largest element of a thread's share of a row: 16-byte vectors t, t +
+// kArgThreads, ... in increasing index order, then single elements past the
+// last whole vector (all of them when the row is not 16-byte aligned). Returns
+// the first element of the largest arg_key (bi < 0: none).
+//
+// 16-bit rows are compared two elements at a time: (magnitude ^ sign) - sign
+// orders them as signed 16-bit integers with -0 equal to +0, so a vector costs
+// 3 packed operations per element pair more than its load, instead of a
+// conversion, a NaN test and a 32-bit key per element; the best vector is kept
+// whole and searched once at the end. NaNs (a magnitude past infinity's) are
+// only detected: `nan` then tells the caller that the result counts numbers
+// only. kArgVec vectors (a 152064-element row's whole share) are in flight at
+// a time; one workgroup reads a row, so its CU's load rate is the bound
+// (26 rows of 152064 bf16 elements: 18.5 us with 32-bit keys and 8 vectors in
+// flight, 12.8 us like this).
+typedef short s16x2_t __attribute__((ext_vector_type(2)));
+constexpr int kArgVec = 10;
+
 template <int DT>
-__device__ int row_argmax(const typename Elem<DT>::T* __restrict__ x, int64_t V, int32_t* out) {
+__device__ __forceinline__ void share_best(const typename Elem<DT>::T* __restrict__ x, int64_t V, int64_t nvec,
+                                           uint32_t& bk, int& bi, bool& nan) {
   typedef typename Elem<DT>::T T;
-  constexpr int kPer = 16 / sizeof(T);  // elements per 16-byte vector
-  constexpr int kVec = 8;               // vectors per thread held in flight
-  uint32_t bk = 0;                      // below every real key
-  int bi = -1;
-  const bool aligned = (((uintptr_t)x) & 15) == 0;
-  const int64_t nvec = aligned ? V / kPer : 0;
-  for (int64_t v0 = 0; v0 < nvec; v0 += (int64_t)kVec * kArgThreads) {
-    u32x4_t buf[kVec];
+  constexpr int kPer = 16 / sizeof(T);
+  bk = 0;  // below every real key
+  bi = -1;
+  nan = false;
+  if constexpr (DT == PE_DTYPE_F32) {
+    for (int64_t v0 = 0; v0 < nvec; v0 += (int64_t)kArgVec * kArgThreads) {
+      u32x4_t buf[kArgVec];
 #pragma unroll
-    for (int k = 0; k < kVec; ++k) {
-      const int64_t vi = v0 + (int64_t)k * kArgThreads + threadIdx.x;
-      if (vi < nvec) buf[k] = *(const u32x4_t*)(x + vi * kPer);
-    }
+      for (int k = 0; k < kArgVec; ++k) {
+        const int64_t vi = v0 + (int64_t)k * kArgThreads + threadIdx.x;
+        if (vi < nvec) buf[k] = *(const u32x4_t*)(x + vi * kPer);
+      }
 #pragma unroll
-    for (int k = 0; k < kVec; ++k) {
-      const int64_t vi = v0 + (int64_t)k * kArgThreads + threadIdx.x;
-      if (vi < nvec) {
-        const T* e = (const T*)&buf[k];
+      for (int k = 0; k < kArgVec; ++k) {
+        const int64_t vi = v0 + (int64_t)k * kArgThreads + threadIdx.x;
+        if (vi < nvec) {
 #pragma unroll
-        for (int j = 0; j < kPer; ++j) {
-          const uint32_t key = arg_key(Elem<DT>::load(e, j));
-          if (key > bk) {
-            bk = key;
-            bi = (int)(vi * kPer + j);
+          for (int j = 0; j < 4; ++j) {
+            const float v = __uint_as_float(buf[k][j]);
+            nan |= v != v;
+            const uint32_t key = arg_key(v);
+            if (key > bk) {
+              bk = key;
+              bi = (int)(vi * kPer + j);
+            }
           }
         }
       }
     }
+  } else {
+    constexpr uint32_t kInf = DT == PE_DTYPE_BF16 ? 0x7f80u : 0x7c00u;
+    int best = -32768, bv = -1;  // below every number's key
+    u32x4_t bw = {0, 0, 0, 0};
+    uint32_t mag = 0;  // packed maximum of the magnitudes
+    typedef unsigned short u16x2_t __attribute__((ext_vector_type(2)));
+    auto key2 = [](uint32_t w) -> s16x2_t {
+      const s16x2_t sg = __builtin_bit_cast(s16x2_t, w) >> 15;
+      return (__builtin_bit_cast(s16x2_t, w & 0x7fff7fffu) ^ sg) - sg;
+    };
+    for (int64_t v0 = 0; v0 < nvec; v0 += (int64_t)kArgVec * kArgThreads) {
+      u32x4_t buf[kArgVec];
+#pragma unroll
+      for (int k = 0; k < kArgVec; ++k) {
+        const int64_t vi = v0 + (int64_t)k * kArgThreads + threadIdx.x;
+        if (vi < nvec) buf[k] = *(const u32x4_t*)(x + vi * kPer);
+      }
+#pragma unroll
+      for (int k = 0; k < kArgVec; ++k) {
+        const int64_t vi = v0 + (int64_t)k * kArgThreads + threadIdx.x;
+        if (vi < nvec) {
+          s16x2_t m = key2(buf[k][0]);
+#pragma unroll
+          for (int j = 1; j < 4; ++j) m = __builtin_elementwise_max(m, key2(buf[k][j]));
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            mag = __builtin_bit_cast(
+                uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2_t, mag),
+                                                    __builtin_bit_cast(u16x2_t, buf[k][j] & 0x7fff7fffu)));
+          const int top = max((int)m[0], (int)m[1]);
+          if (top > best) {
+            best = top;
+            bv = (int)vi;
+            bw = buf[k];
+          }
+        }
+      }
+    }
+    nan = (mag & 0xffffu) > kInf || (mag >> 16) > kInf;
+    if (bv >= 0) {
+#pragma unroll
+      for (int j = 3; j >= 0; --j) {
+        const s16x2_t m = key2(bw[j]);
+        if (m[1] == best) bi = bv * kPer + 2 * j + 1;
+        if (m[0] == best) bi = bv * kPer + 2 * j;
+      }
+      // the winner's own 32-bit key
+      uint32_t e = bw[0];
+#pragma unroll
+      for (int j = 1; j < 4; ++j) e = ((bi >> 1) & 3) == j ? bw[j] : e;
+      const uint16_t bits = (uint16_t)((bi & 1) ? e >> 16 : e);
+      bk = arg_key(Elem<DT>::load(&bits, 0));
+    }
   }
   for (int64_t i = nvec * kPer + threadIdx.x; i < V; i += kArgThreads) {
-    const uint32_t key = arg_key(Elem<DT>::load(x, i));
+    const float v = Elem<DT>::load(x, i);
+    nan |= v != v;
+    const uint32_t key = arg_key(v);
     if (key > bk) {
       bk = key;
       bi = (int)i;
+    }
+  }
+}
+
+// Whole 16-byte vectors of a row (none when it is not 16-byte aligned).
+template <int DT>
+__device__ __forceinline__ int64_t row_vectors(const typename Elem<DT>::T* x, int64_t V) {
+  return (((uintptr_t)x) & 15) == 0 ? V / (16 / (int64_t)sizeof(typename Elem<DT>::T)) : 0;
+}
+
+// One block of kArgThreads per row: every thread's best, then the block's with
+// (key descending, index ascending). A row with a NaN is searched again for
+// its first NaN (every NaN has the largest key).
+template <int DT>
+__device__ int row_argmax(const typename Elem<DT>::T* __restrict__ x, int64_t V, int32_t* out) {
+  uint32_t bk;
+  int bi;
+  bool nan;
+  share_best<DT>(x, V, row_vectors<DT>(x, V), bk, bi, nan);
+  if (__syncthreads_or(nan)) {
+    bk = 0;
+    bi = -1;
+    for (int64_t i = threadIdx.x; i < V; i += kArgThreads) {
+      const uint32_t key = arg_key(Elem<DT>::load(x, i));
+      if (key > bk) {
+        bk = key;
+        bi = (int)i;
+      }
     }
   }
   auto better = [](uint32_t k2, int i2, uint32_t k1, int i1) {  // (k2, i2) beats (k1, i1)
@@ -383,19 +482,34 @@ __global__ void kv_gather_kernel(uint8_t* __restrict__ kc, uint8_t* __restrict__
   }
 }
 
-// Beam tree proposal (propose_tree, src/pe/decode/tree.py:34-55) in two
-// launches. draft_topk_kernel: one block per depth row computes the row's
-// log-sum-exp in fp32 and selects the row's top c_d tokens one at a time, each
-// round the best element after the previous one in (value descending, index
-// ascending) order; the winners' log-probabilities (x - max) - log(sum) go to
-// scratch. beam_kernel: one block walks the depths; candidate (parent p, rank
-// j in the row) scores cum[p] + lp[j] in float64, and its position in the
-// stable descending order of the candidate list (parent-major, as the
-// reference builds it) is counted directly: j for its own parent, plus, for
-// every other parent, the candidates that score higher (or equal, for parents
-// before it), found by binary search since each parent's scores do not
-// increase with j.
+// Beam tree proposal (propose_tree, src/pe/decode/tree.py:34-55) in three
+// launches.
+//   * draft_topk_kernel: one block per depth row. Every thread finds the best
+//     element of its share of the row; one wave then takes the row's top c_d
+//     tokens in (value descending, index ascending) order: the best of the
+//     1024 shares, whose owner's share (about V / 1024 elements, read across
+//     the wave) is searched for its next best. Streaming the row again for
+//     every token took 199 us for five rows of 152064 at five tokens each;
+//     this takes 20 us (a row is one CU's 304 KB), the sums below 8.
+//   * draft_expsum_kernel: the row's sum of exp(x - max) in fp32. The sum keeps
+//     the order of 1024 strided partial sums (element i in partial i % 1024,
+//     increasing i), the partials of 64 neighbours added by a butterfly: block
+//     s owns the 64 partials of slice s and computes their exponentials in
+//     parallel, one wave adds them up in order. (Sums of equal logits over
+//     different rows tie up to these roundings, so the order decides trees.)
+//   * beam_kernel: logarithms of the rows' sums (slices in order), the
+//     candidates' log-probabilities (x - max) - log(sum), then one block walks
+//     the depths; candidate (parent p, rank j in the row) scores cum[p] +
+//     lp[j] in float64, and its position in the stable descending order of the
+//     candidate list (parent-major, as the reference builds it) is counted
+//     directly: j for its own parent, plus, for every other parent, the
+//     candidates that score higher (or equal, for parents before it), found by
+//     binary search since each parent's scores do not increase with j.
 constexpr int kBeamThreads = 256;
+constexpr int kSlices = kArgThreads / 64;  // slices of 64 partial sums
+constexpr int kExpTile = 128;              // elements of a partial sum staged at a time
+constexpr int kExpThreads = 512;
+static_assert(kSlices <= PE_PROPOSE_MAX_WIDTH, "a row's slice sums are staged in its log-probability scratch");
 
 struct BeamShape {
   int k;
@@ -410,8 +524,8 @@ __device__ __forceinline__ bool key_before(uint32_t k2, int i2, uint32_t k1, int
   return k2 > k1 || (k2 == k1 && i2 < i1);
 }
 
-// block-wide (key, index) reduction over kArgThreads threads; every thread gets the result
-__device__ void block_best(uint32_t& bk, int& bi, uint32_t* wk, int* wi) {
+// wave-wide (key, index) reduction; every lane gets the result
+__device__ __forceinline__ void wave_best(uint32_t& bk, int& bi) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
     const uint32_t k2 = __shfl_xor(bk, o, 64);
@@ -421,105 +535,167 @@ __device__ void block_best(uint32_t& bk, int& bi, uint32_t* wk, int* wi) {
       bi = i2;
     }
   }
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) {
-    wk[threadIdx.x >> 6] = bk;
-    wi[threadIdx.x >> 6] = bi;
-  }
-  __syncthreads();
-  bk = wk[0];
-  bi = wi[0];
-  for (int w = 1; w < kArgThreads / 64; ++w)
-    if (key_before(wk[w], wi[w], bk, bi)) {
-      bk = wk[w];
-      bi = wi[w];
-    }
 }
 
-__device__ float block_sum(float v, float* ws) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) ws[threadIdx.x >> 6] = v;
-  __syncthreads();
-  float s = 0.f;
-  for (int w = 0; w < kArgThreads / 64; ++w) s += ws[w];
-  return s;
-}
-
+// A row with a NaN, without a finite value or with +inf flags PE_ERR_VALUE and
+// leaves token -1 in its first place.
 template <int DT>
 __global__ __launch_bounds__(kArgThreads) void draft_topk_kernel(const typename Elem<DT>::T* __restrict__ logits,
                                                                  int64_t ld, int64_t V, BeamShape bs,
-                                                                 float* __restrict__ lp_out,
                                                                  int32_t* __restrict__ tok_out, int32_t* status) {
   const int d = blockIdx.x;
   const typename Elem<DT>::T* x = logits + (int64_t)d * ld;
-  __shared__ uint32_t wk[kArgThreads / 64];
-  __shared__ int wi[kArgThreads / 64];
-  __shared__ float ws[kArgThreads / 64];
-  // the row maximum (the first selection round) and NaN detection
-  uint32_t bk = 0;
-  int bi = -1;
-  int nan = 0;
-  for (int64_t i = threadIdx.x; i < V; i += kArgThreads) {
-    const float v = Elem<DT>::load(x, i);
-    nan |= v != v;
-    const uint32_t key = arg_key(v);
-    if (key_before(key, (int)i, bk, bi)) {
-      bk = key;
-      bi = (int)i;
-    }
-  }
+  constexpr int kPer = 16 / sizeof(typename Elem<DT>::T);
+  const int64_t nvec = row_vectors<DT>(x, V);
+  __shared__ uint32_t s_key[kArgThreads];
+  __shared__ int s_idx[kArgThreads];
+  uint32_t bk;
+  int bi;
+  bool nan;
+  share_best<DT>(x, V, nvec, bk, bi, nan);
+  s_key[threadIdx.x] = bk;
+  s_idx[threadIdx.x] = bi;
   nan = __syncthreads_or(nan);
-  block_best(bk, bi, wk, wi);
-  const float mx = Elem<DT>::load(x, bi);
-  if (nan || !(mx > -INFINITY) || mx == INFINITY) {
-    if (threadIdx.x == 0 && status) atomicOr(status, PE_ERR_VALUE);
-    return;
-  }
-  float s = 0.f;
-  for (int64_t i = threadIdx.x; i < V; i += kArgThreads) s += expf(Elem<DT>::load(x, i) - mx);
-  const float logsum = logf(block_sum(s, ws));
-  const int c = bs.cand[d];
-  for (int j = 0;; ++j) {
-    if (threadIdx.x == 0) {
-      lp_out[d * PE_PROPOSE_MAX_WIDTH + j] = (Elem<DT>::load(x, bi) - mx) - logsum;
-      tok_out[d * PE_PROPOSE_MAX_WIDTH + j] = bi;
-    }
-    if (j + 1 >= c) break;
-    // next round: the best element after (bk, bi) in the order
-    const uint32_t pk = bk;
-    const int pi = bi;
-    bk = 0;
-    bi = -1;
-    for (int64_t i = threadIdx.x; i < V; i += kArgThreads) {
-      const uint32_t key = arg_key(Elem<DT>::load(x, i));
-      if (key_before(pk, pi, key, (int)i) && key_before(key, (int)i, bk, bi)) {
-        bk = key;
-        bi = (int)i;
+  if (threadIdx.x >= 64) return;
+  const int lane = threadIdx.x;
+  int32_t* out = tok_out + d * PE_PROPOSE_MAX_WIDTH;
+  // the best of this lane's 16 shares (lane, lane + 64, ...)
+  uint32_t lk = 0;
+  int li = -1;
+  auto scan = [&]() {
+    lk = 0;
+    li = -1;
+#pragma unroll
+    for (int q = 0; q < kArgThreads / 64; ++q) {
+      const uint32_t k2 = s_key[lane + 64 * q];
+      const int i2 = s_idx[lane + 64 * q];
+      if (key_before(k2, i2, lk, li)) {
+        lk = k2;
+        li = i2;
       }
     }
-    block_best(bk, bi, wk, wi);
+  };
+  scan();
+  const int c = bs.cand[d];
+  for (int j = 0; j < c; ++j) {
+    uint32_t pk = lk;
+    int pi = li;
+    wave_best(pk, pi);
+    if (j == 0) {
+      const float mx = Elem<DT>::load(x, pi);
+      if (nan || !(mx > -INFINITY) || mx == INFINITY) {
+        if (lane == 0) {
+          out[0] = -1;
+          if (status) atomicOr(status, PE_ERR_VALUE);
+        }
+        return;
+      }
+    }
+    if (lane == 0) out[j] = pi;
+    if (j + 1 == c) break;
+    // the owner's next best after (pk, pi)
+    const bool in_vec = pi < nvec * kPer;
+    const int owner = (int)((in_vec ? pi / kPer : pi - nvec * kPer) % kArgThreads);
+    const int64_t nv = nvec > owner ? (nvec - owner + kArgThreads - 1) / kArgThreads : 0;
+    uint32_t k1 = 0;
+    int i1 = -1;
+    auto offer = [&](int64_t i) {
+      const uint32_t key = arg_key(Elem<DT>::load(x, i));
+      if (key_before(pk, pi, key, (int)i) && key_before(key, (int)i, k1, i1)) {
+        k1 = key;
+        i1 = (int)i;
+      }
+    };
+#pragma unroll 4
+    for (int64_t q = lane; q < nv * kPer; q += 64) offer((owner + (q / kPer) * kArgThreads) * kPer + q % kPer);
+    for (int64_t i = nvec * kPer + owner + (int64_t)lane * kArgThreads; i < V; i += 64 * kArgThreads) offer(i);
+    wave_best(k1, i1);
+    if (lane == (owner & 63)) {
+      s_key[owner] = k1;
+      s_idx[owner] = i1;
+      scan();
+    }
   }
 }
 
-__global__ __launch_bounds__(kBeamThreads) void beam_kernel(BeamShape bs, const float* __restrict__ lp,
+// grid (kSlices, depth rows)
+template <int DT>
+__global__ __launch_bounds__(kExpThreads) void draft_expsum_kernel(const typename Elem<DT>::T* __restrict__ logits,
+                                                                   int64_t ld, int64_t V,
+                                                                   const int32_t* __restrict__ tok,
+                                                                   float* __restrict__ sums) {
+  const int slice = blockIdx.x, d = blockIdx.y;
+  const typename Elem<DT>::T* x = logits + (int64_t)d * ld;
+  const int first = tok[d * PE_PROPOSE_MAX_WIDTH];
+  if (first < 0) return;  // an invalid row (the whole block leaves)
+  const float mx = Elem<DT>::load(x, first);
+  __shared__ float e[kExpTile][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t part = slice * 64 + lane;
+  const int64_t n = part < V ? (V - part + kArgThreads - 1) / kArgThreads : 0;  // this lane's elements
+  const int64_t most = slice * 64 < V ? (V - slice * 64 + kArgThreads - 1) / kArgThreads : 0;
+  float s = 0.f;
+  for (int64_t j0 = 0; j0 < most; j0 += kExpTile) {
+    const int64_t j1 = min(most, j0 + kExpTile);
+#pragma unroll 4
+    for (int64_t j = j0 + wave; j < j1; j += kExpThreads / 64)
+      if (j < n) e[j - j0][lane] = expf(Elem<DT>::load(x, part + j * kArgThreads) - mx);
+    __syncthreads();
+    if (wave == 0) {
+      const int64_t m = min(n, j1) - j0;
+#pragma unroll 8
+      for (int64_t j = 0; j < m; ++j) s += e[j][lane];
+    }
+    __syncthreads();
+  }
+  if (wave != 0) return;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+  if (lane == 0) sums[d * PE_PROPOSE_MAX_WIDTH + slice] = s;
+}
+
+// lp: the rows' slice sums on entry, their candidates' log-probabilities on return.
+template <int DT>
+__global__ __launch_bounds__(kBeamThreads) void beam_kernel(const typename Elem<DT>::T* __restrict__ logits,
+                                                            int64_t ld, BeamShape bs, float* __restrict__ lp,
                                                             const int32_t* __restrict__ tok,
                                                             int64_t* __restrict__ node_tokens,
                                                             int32_t* __restrict__ parents, const int32_t* status) {
-  if (status && *status & PE_ERR_VALUE) return;
+  __shared__ float s_sum[PE_PROPOSE_MAX_DEPTH][kSlices];
+  __shared__ float s_lp[PE_PROPOSE_MAX_DEPTH][PE_PROPOSE_MAX_WIDTH];
+  __shared__ int s_tok[PE_PROPOSE_MAX_DEPTH][PE_PROPOSE_MAX_WIDTH];
   __shared__ double cum[PE_PROPOSE_MAX_WIDTH], ncum[PE_PROPOSE_MAX_WIDTH], row[PE_PROPOSE_MAX_WIDTH];
   __shared__ int node[PE_PROPOSE_MAX_WIDTH];
+  int bad = status && (*status & PE_ERR_VALUE);
+  for (int i = threadIdx.x; i < bs.k * PE_PROPOSE_MAX_WIDTH; i += kBeamThreads) {
+    const int d = i / PE_PROPOSE_MAX_WIDTH, j = i % PE_PROPOSE_MAX_WIDTH;
+    if (j < kSlices) s_sum[d][j] = lp[i];
+    if (j < bs.cand[d]) s_tok[d][j] = tok[i];
+    if (j == 0) bad |= tok[i] < 0;
+  }
+  if (__syncthreads_or(bad)) return;
+  for (int i = threadIdx.x; i < bs.k * PE_PROPOSE_MAX_WIDTH; i += kBeamThreads) {
+    const int d = i / PE_PROPOSE_MAX_WIDTH, j = i % PE_PROPOSE_MAX_WIDTH;
+    if (j >= bs.cand[d]) continue;
+    const typename Elem<DT>::T* x = logits + (int64_t)d * ld;
+    const float mx = Elem<DT>::load(x, s_tok[d][0]);
+    float s = 0.f;
+    for (int w = 0; w < kSlices; ++w) s += s_sum[d][w];
+    const float v = (Elem<DT>::load(x, s_tok[d][j]) - mx) - logf(s);
+    s_lp[d][j] = v;
+    lp[i] = v;
+  }
   int nb = 1, base = 0;
   if (threadIdx.x == 0) {
     cum[0] = 0.0;
     node[0] = -1;
   }
+  __syncthreads();
   for (int d = 0; d < bs.k; ++d) {
     const int c = bs.cand[d];
     const int n = nb * c;
     const int kept = min(bs.width[d], n);
-    if (threadIdx.x < c) row[threadIdx.x] = (double)lp[d * PE_PROPOSE_MAX_WIDTH + threadIdx.x];
+    if (threadIdx.x < c) row[threadIdx.x] = (double)s_lp[d][threadIdx.x];
     __syncthreads();
     for (int q = threadIdx.x; q < n; q += kBeamThreads) {
       const int p = q / c, j = q - p * c;
@@ -541,7 +717,7 @@ __global__ __launch_bounds__(kBeamThreads) void beam_kernel(BeamShape bs, const 
       }
       if (r < kept) {
         ncum[r] = sc;
-        node_tokens[base + r] = tok[d * PE_PROPOSE_MAX_WIDTH + j];
+        node_tokens[base + r] = s_tok[d][j];
         parents[base + r] = node[p];
       }
     }
@@ -771,22 +947,23 @@ extern "C" int pe_propose_tree(const void* logits, int64_t ld, int k, int64_t V,
   float* lp = (float*)scratch;
   int32_t* tok = (int32_t*)((char*)scratch + (size_t)k * PE_PROPOSE_MAX_WIDTH * sizeof(float));
   hipStream_t st = (hipStream_t)stream;
+#define PE_PROPOSE(D)                                                                                            \
+  do {                                                                                                          \
+    const Elem<D>::T* x = (const Elem<D>::T*)logits;                                                            \
+    draft_topk_kernel<D><<<k, kArgThreads, 0, st>>>(x, ld, V, bs, tok, status);                                  \
+    PE_CHECK_LAUNCH();                                                                                          \
+    draft_expsum_kernel<D><<<dim3(kSlices, k), kExpThreads, 0, st>>>(x, ld, V, tok, lp);                         \
+    PE_CHECK_LAUNCH();                                                                                          \
+    beam_kernel<D><<<1, kBeamThreads, 0, st>>>(x, ld, bs, lp, tok, node_tokens, parents, status);                \
+    PE_CHECK_LAUNCH();                                                                                          \
+  } while (0)
   switch (dtype) {
-    case PE_DTYPE_F32:
-      draft_topk_kernel<PE_DTYPE_F32><<<k, kArgThreads, 0, st>>>((const float*)logits, ld, V, bs, lp, tok, status);
-      break;
-    case PE_DTYPE_BF16:
-      draft_topk_kernel<PE_DTYPE_BF16><<<k, kArgThreads, 0, st>>>((const uint16_t*)logits, ld, V, bs, lp, tok, status);
-      break;
-    case PE_DTYPE_F16:
-      draft_topk_kernel<PE_DTYPE_F16><<<k, kArgThreads, 0, st>>>((const uint16_t*)logits, ld, V, bs, lp, tok, status);
-      break;
-    default:
-      return PE_ERR_ARG;
+    case PE_DTYPE_F32: PE_PROPOSE(PE_DTYPE_F32); break;
+    case PE_DTYPE_BF16: PE_PROPOSE(PE_DTYPE_BF16); break;
+    case PE_DTYPE_F16: PE_PROPOSE(PE_DTYPE_F16); break;
+    default: return PE_ERR_ARG;
   }
-  PE_CHECK_LAUNCH();
-  beam_kernel<<<1, kBeamThreads, 0, st>>>(bs, lp, tok, node_tokens, parents, status);
-  PE_CHECK_LAUNCH();
+#undef PE_PROPOSE
   return PE_OK;
 }
 
