@@ -752,9 +752,9 @@ constexpr int kBigTab = 16 * 64 * 4;          // one producer's table: 16 codes 
 constexpr int kBigBufUnit = kBigNT * 8 * 64 * 16;  // B fragments of one unit: 4 tiles x 8 k-steps x 64 lanes x 16 B
 constexpr int kBigSmem = kWaves * kBigTab + 2 * kBigBufUnit;
 
-template <int WV>
+template <int WV, bool AF>
 __device__ __forceinline__ void bigws_producer(uint8_t* smem, const uint8_t* __restrict__ W,
-                                               const uint16_t* __restrict__ Wabs, int NP, int group, int u0, int u1) {
+                                               const void* __restrict__ Wabs, int NP, int group, int u0, int u1) {
   const int n = u1 - u0;
   const int lane = threadIdx.x & 63;
   constexpr int TB = WV * kBigTab;  // this wave's table
@@ -769,7 +769,10 @@ __device__ __forceinline__ void bigws_producer(uint8_t* smem, const uint8_t* __r
     q[0] = __builtin_nontemporal_load(wp);
     q[1] = __builtin_nontemporal_load(wp + 64);
   };
-  auto load_abs = [&](int p) -> uint32_t { return (uint32_t)Wabs[(tile * NP + min(p, u1 - 1)) * 64 + lane]; };
+  auto load_abs = [&](int p) -> uint32_t {
+    const int64_t i = (tile * NP + min(p, u1 - 1)) * 64 + lane;
+    return AF ? ((const uint32_t*)Wabs)[i] : (uint32_t)((const uint16_t*)Wabs)[i];
+  };
   // relative unit t (table half SL) into ring slot t % 2
   auto dequant = [&](const u32x4_t (&q)[2], int t, auto slot_c) {
     constexpr int SL = decltype(slot_c)::value;
@@ -800,7 +803,7 @@ __device__ __forceinline__ void bigws_producer(uint8_t* smem, const uint8_t* __r
   uint32_t a0 = load_abs(u0), a1 = load_abs(u0 + 1);
   for (int r = 0; r <= n; r += 2) {
     if (r < n) {
-      nf4_build_table2<TB, false>(lanetab, a0, a1);  // the reads of units r - 2, r - 1 are issued
+      nf4_build_table2<TB, AF>(lanetab, a0, a1);  // the reads of units r - 2, r - 1 are issued
       a0 = load_abs(u0 + r + 2);
       a1 = load_abs(u0 + r + 3);
       dequant(qa, r, kLo);
@@ -928,10 +931,10 @@ __device__ __forceinline__ void bigws_consumer(uint8_t* smem, const uint16_t* __
 
 constexpr int kWsWaves = 2 * kWaves;  // producers + consumers
 
-template <bool SW>
+template <bool SW, bool AF>
 __global__ __launch_bounds__(kWsWaves * 64, 1) void nf4_gemm_bigws_kernel(const uint16_t* __restrict__ X,
                                                                           const uint8_t* __restrict__ W,
-                                                                          const uint16_t* __restrict__ Wabs, int NP,
+                                                                          const void* __restrict__ Wabs, int NP,
                                                                           int pps, int mtiles, EpiArgs e) {
   __shared__ __align__(256) uint8_t smem[kBigSmem];
   const int group = blockIdx.x, split = blockIdx.y;
@@ -940,17 +943,17 @@ __global__ __launch_bounds__(kWsWaves * 64, 1) void nf4_gemm_bigws_kernel(const 
   if (u0 >= u1) return;  // a whole workgroup: no barrier is left waiting
   if (wave < kWaves) {
     switch (wave) {
-      case 0: bigws_producer<0>(smem, W, Wabs, NP, group, u0, u1); break;
-      case 1: bigws_producer<1>(smem, W, Wabs, NP, group, u0, u1); break;
-      case 2: bigws_producer<2>(smem, W, Wabs, NP, group, u0, u1); break;
-      default: bigws_producer<3>(smem, W, Wabs, NP, group, u0, u1); break;
+      case 0: bigws_producer<0, AF>(smem, W, Wabs, NP, group, u0, u1); break;
+      case 1: bigws_producer<1, AF>(smem, W, Wabs, NP, group, u0, u1); break;
+      case 2: bigws_producer<2, AF>(smem, W, Wabs, NP, group, u0, u1); break;
+      default: bigws_producer<3, AF>(smem, W, Wabs, NP, group, u0, u1); break;
     }
     return;
   }
   // the consumers (the critical path) win issue arbitration over the
   // producers of their SIMD
   __builtin_amdgcn_s_setprio(2);
-  // grid.z: blocks of eight 32-row tiles (a prefill of more than 256 rows)
+  // grid.z: blocks of eight 32-row tiles (more than 256 rows)
   const int mt0 = blockIdx.z * 8 + (wave - kWaves) * 2;
   const int nmt = max(0, min(2, mtiles - mt0));
   if (nmt == 2) bigws_consumer<2, SW>(smem, X, NP, group, u0, u1, mt0, e, split);
@@ -1098,9 +1101,9 @@ __global__ __launch_bounds__(kWaves * 64, 2) void dense_gemm_bigm_kernel(const u
 // One workgroup = 4 waves = a block of up to 256 rows (32-row tiles of the
 // A-tiled X) x 256 columns (eight 32-column weight tiles); wave w owns the
 // row tiles MI (w / 2) .. + MI - 1 and the columns 128 (w % 2) .. + 127: MI x 4
-// MFMA tiles (MI = 4: 256 fp32 accumulators). The last row block of a launch
-// runs MI = 2 or 1 when it holds at most four or two tiles (777 rows: 3 x 256
-// + 9, the 9 rows at the price of 64).
+// MFMA tiles (MI = 4: 256 fp32 accumulators). A block of fewer tiles, the last
+// of a launch or all of a small one, runs MI = 3, 2 or 1 (777 rows: 3 x 256 +
+// 9, the 9 rows at the price of 64).
 //
 // K is walked in stages of two MFMA k-steps. A stage's 4 MI A fragments and 16
 // B fragments, 1 KiB each, go straight from global memory into an LDS ring of
@@ -1135,7 +1138,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void dense_gemm_bigm_kernel(const u
 constexpr int kEpiT16 = 0, kEpiTF32 = 1, kEpiTSwiglu = 2;
 constexpr int kT256Smem = 144 * 1024;
 constexpr int t256_stage(int MI) { return (4 * MI + 16) * 1024; }
-constexpr int t256_ring(int MI) { return kT256Smem / t256_stage(MI); }  // 4, 6 and 7 stages
+constexpr int t256_ring(int MI) { return kT256Smem / t256_stage(MI); }  // 4, 5, 6 and 7 stages
 // s_waitcnt immediate: vmcnt = n, lgkmcnt = 0, expcnt at its maximum
 constexpr int wait_vm_lgkm0(int n) { return (n & 15) | (7 << 4) | ((n >> 4) << 14); }
 
@@ -1143,7 +1146,7 @@ struct T256Args {
   const uint16_t* x;
   const uint16_t* w;
   int units, ups;      // 128-wide K units: all, and per split
-  int mtiles, mblocks, bt; // 32-row tiles, and blocks of bt (8, 4 or 2) of them
+  int mtiles, mblocks, bt; // 32-row tiles, and blocks of bt (8, 6, 4 or 2) of them
   int M;
   void* out;
   int64_t ld;     // row stride of out in elements (16-bit and fp32 outputs)
@@ -1174,18 +1177,16 @@ __device__ __forceinline__ void t256_tile(uint8_t* smem, const T256Args& p, int 
     }
   }
   // fragments i0 .. i1 - 1 of stage t (past the end: the last one again) into ring slot `slot`
-  auto issue = [&](int t, int slot, auto i0, auto i1) {
+  auto issue = [&](int t, int slot, int i0, int i1) {
     const int tt = u0 * 4 + min(t, nst - 1);
     const uint8_t* xs = xb + (int64_t)tt * 2048;
     const uint8_t* ws = wb + (int64_t)(8 * (tt >> 2) + (tt & 3)) * 1024;
     const uint32_t dst = lds_base + slot * STG + wave * (PW * 1024);
 #pragma unroll
-    for (int i = decltype(i0)::value; i < decltype(i1)::value; ++i)
+    for (int i = i0; i < i1; ++i)
       lds_dma16(wave * PW + i < AF ? (const void*)xs : (const void*)ws, voff[i],
                 __builtin_amdgcn_readfirstlane(dst + i * 1024));
   };
-  constexpr std::integral_constant<int, 0> kFirst{};
-  constexpr std::integral_constant<int, PW> kAll{};
   const int wm = wave >> 1, wn = wave & 1;
   f32x16_t acc[MI][4];
 #pragma unroll
@@ -1207,7 +1208,7 @@ __device__ __forceinline__ void t256_tile(uint8_t* smem, const T256Args& p, int 
                                     : mfma16<DT>(fb[sl][ni], fa[sl][mi], acc[mi][ni]);
   };
 #pragma unroll
-  for (int t = 0; t < R - 1; ++t) issue(t, t, kFirst, kAll);
+  for (int t = 0; t < R - 1; ++t) issue(t, t, 0, PW);
   __builtin_amdgcn_s_waitcnt(wait_vm_lgkm0((R - 2) * PW));
   lds_barrier();
 #pragma unroll
@@ -1224,14 +1225,7 @@ __device__ __forceinline__ void t256_tile(uint8_t* smem, const T256Args& p, int 
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int f = mi * (4 + MI) / MI; f < (mi + 1) * (4 + MI) / MI; ++f) read(st, 1, f);
-      if constexpr (MI == 4) {
-        if (mi == 0) issue(t + R - 1, free_slot, kFirst, std::integral_constant<int, 2>{});
-        if (mi == 1) issue(t + R - 1, free_slot, std::integral_constant<int, 2>{}, std::integral_constant<int, 4>{});
-        if (mi == 2) issue(t + R - 1, free_slot, std::integral_constant<int, 4>{}, std::integral_constant<int, 6>{});
-        if (mi == 3) issue(t + R - 1, free_slot, std::integral_constant<int, 6>{}, kAll);
-      } else if (mi == 0) {
-        issue(t + R - 1, free_slot, kFirst, kAll);
-      }
+      issue(t + R - 1, free_slot, mi * PW / MI, (mi + 1) * PW / MI);
       mul(0, mi);
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -1329,7 +1323,8 @@ __global__ __launch_bounds__(256, 1) void dense_gemm_t256_kernel(T256Args p) {
   const int u0 = split * p.ups, u1 = min(p.units, u0 + p.ups);
   if (u0 >= u1) return;
   const int left = min(p.bt, p.mtiles - mblock * p.bt);
-  if (left > 4) t256_tile<DT, 4, EPI>(smem, p, ntile, mblock, split, u0, (u1 - u0) * 4);
+  if (left > 6) t256_tile<DT, 4, EPI>(smem, p, ntile, mblock, split, u0, (u1 - u0) * 4);
+  else if (left > 4) t256_tile<DT, 3, EPI>(smem, p, ntile, mblock, split, u0, (u1 - u0) * 4);
   else if (left > 2) t256_tile<DT, 2, EPI>(smem, p, ntile, mblock, split, u0, (u1 - u0) * 4);
   else t256_tile<DT, 1, EPI>(smem, p, ntile, mblock, split, u0, (u1 - u0) * 4);
 }
@@ -1952,13 +1947,14 @@ int pe_internal_swiglu_partials(const float* partial, int S, int M, int N, void*
   return PE_OK;
 }
 
-// The many-row NF4 GEMM (A-tiled X of M rows, 64 < M <= 256, N % 128 == 0):
-// split partials [S][M][N]; S chosen for about two workgroups per CU.
+// The many-row NF4 GEMM (A-tiled X of M rows, N % 128 == 0): split partials
+// [S][M][N]; the S splits, the column groups and the blocks of 256 rows fill at
+// most one round of one workgroup per CU.
 namespace {
 struct BigPlan {
   int groups, units, S, pps;
 };
-BigPlan big_plan(int N, int K) {
+BigPlan big_plan(int M, int N, int K) {
   BigPlan p;
   p.groups = N / (32 * kBigNT);
   p.units = K / 128;
@@ -1969,7 +1965,7 @@ BigPlan big_plan(int N, int K) {
   // takes one split).
   static const int forced = env_int("PE_BIGM_SPLITS", 0);
   const int cu = cu_count();
-  int S = cu / p.groups;
+  int S = cu / (p.groups * ((M + 255) / 256));
   if (S < 1) S = 1;
   if (forced > 0) S = forced;
   if (S > kMaxSplits) S = kMaxSplits;
@@ -1980,11 +1976,6 @@ BigPlan big_plan(int N, int K) {
   return p;
 }
 }  // namespace
-
-int64_t pe_internal_nf4_bigm_partials_bytes(int M, int N, int K) {
-  if (M <= 0 || N <= 0 || K < 128 || N % (32 * kBigNT) || K % 128) return 0;
-  return (int64_t)big_plan(N, K).S * M * N * 4;
-}
 
 namespace {
 // Rows per workgroup (32 bt) and K splits of a t256 launch, by its estimated
@@ -1998,11 +1989,11 @@ struct T256Plan {
 };
 T256Plan t256_plan(int M, int N, int K, int max_splits, bool f32_out) {
   constexpr double kFixed = 5.0;
-  auto stage_us = [](int tiles) { return tiles > 4 ? 0.80 : tiles > 2 ? 0.50 : 0.31; };
+  auto stage_us = [](int tiles) { return tiles > 6 ? 0.80 : tiles > 4 ? 0.65 : tiles > 2 ? 0.50 : 0.31; };
   const int mt = (M + 31) / 32, units = K / 128, cu = cu_count();
   T256Plan best = {8, 1};
   double best_t = 1e30;
-  for (int bt = 8; bt >= 2; bt >>= 1) {
+  for (int bt = 8; bt >= 2; bt -= 2) {
     const int full = mt / bt, rem = mt % bt;
     for (int S = 1; S <= max_splits && S <= units; ++S) {
       const int ups = (units + S - 1) / S;
@@ -2058,28 +2049,30 @@ int t256_launch(const void* x_tiled, int M, int K, const void* w, int dtype, int
 }
 }  // namespace
 
-// The SwiGLU linear over many rows (N interleaved gate / up columns), the
-// activation stored A-tiled; PE_ERR_ARG for shapes without whole column tiles.
-bool pe_internal_dense_swiglu_fits(int M, int N, int K) { return K % 128 == 0 && t256_shape(M, N, K); }
-int pe_internal_dense_swiglu(const void* x_tiled, int M, int K, const void* w, int dtype, int N, void* act,
-                             int out_units, hipStream_t st) {
-  if (!x_tiled || !w || !act || M <= 0 || !pe_internal_dense_swiglu_fits(M, N, K) || out_units * 256 != N)
-    return PE_ERR_ARG;
-  return t256_launch(x_tiled, M, K, w, dtype, N, act, 0, kEpiTSwiglu, out_units, t256_plan(M, N, K, 1, false), st);
+namespace {
+// K splits of pe_internal_dense_bigm's fp32 partials.
+int dense_bigm_splits(int M, int N, int K, int max_splits) {
+  if (t256_shape(M, N, K)) return t256_plan(M, N, K, max_splits, true).S;
+  const int np = K / 128, mblocks = (M + 255) / 256;
+  return max_splits >= 2 && (int64_t)(N / (32 * kBigNT)) * mblocks < 512 && np >= 4 ? 2 : 1;
 }
+}  // namespace
 
 // splits: null, or receives the K splits of the fp32 partials, at most max_splits
 int pe_internal_dense_bigm(const void* x_tiled, int M, int K, const void* w, int dtype, int N, void* out,
                            int64_t ld_out, hipStream_t st, bool f32_out, int* splits, int max_splits) {
   if (!x_tiled || !w || !out || M <= 0 || K % 128 || N % (32 * kBigNT) || ld_out < N) return PE_ERR_ARG;
   if (splits) *splits = 1;
-  // More than one row block: 256-column tiles from the LDS ring (M = 300, N =
-  // K = 4096: 39 against 72 us with the 128-column kernel; 1500 rows, K =
-  // 11008: 176 against 203; 777 rows of the 152064-column lm_head 1.2 against
-  // 1.7 ms). At most 256 rows of a wide lm_head are bound by its weights, read
-  // by twice as many workgroups in the 128-column kernel (208 rows: 433
-  // against 464 us).
-  if (M > 256 && t256_shape(M, N, K)) {
+  // 256-column tiles from the LDS ring; the 128-column kernel keeps widths that
+  // are not a multiple of 256 (M = 300, N = K = 4096: 39 against 72 us; 1500
+  // rows, K = 11008: 176 against 203; the 152064-column lm_head over 70, 160
+  // and 777 rows 317, 356 and 1190 us against 352, 407 and 1742). Seven row
+  // tiles under a lm_head of more than a round of tiles stay there too: the
+  // padded eighth tile is an eighth more matrix-core work at full power, and in
+  // the batched pass (208 x 152064 x 5120, back to back) it cost 35 us (a lone
+  // launch: 411 against 433; 208 x 32000 x 4096, half a round: 70 against 87).
+  const bool padded = !f32_out && (M + 31) / 32 == 7 && N / 256 > cu_count();
+  if (t256_shape(M, N, K) && !padded) {
     const T256Plan plan = t256_plan(M, N, K, splits && f32_out ? max_splits : 1, f32_out);
     if (splits) *splits = plan.S;
     return t256_launch(x_tiled, M, K, w, dtype, N, out, ld_out, f32_out ? kEpiTF32 : kEpiT16, 0, plan, st);
@@ -2088,9 +2081,7 @@ int pe_internal_dense_bigm(const void* x_tiled, int M, int K, const void* w, int
   const int mtiles = (M + 31) / 32;
   // fp32 partials for a caller that sums splits: two K splits when the column
   // groups x row blocks would fill fewer than two workgroups per CU
-  int S = 1;
-  if (f32_out && splits && max_splits >= 2 && (int64_t)(N / (32 * kBigNT)) * ((mtiles + 7) / 8) < 512 && np >= 4)
-    S = 2;
+  const int S = f32_out && splits ? dense_bigm_splits(M, N, K, max_splits) : 1;
   if (splits) *splits = S;
   const dim3 grid(N / (32 * kBigNT), (mtiles + 7) / 8, S);
 #define PE_DBIGM_LAUNCH(D, F)                                                                             \
@@ -2111,68 +2102,77 @@ int pe_internal_dense_bigm(const void* x_tiled, int M, int K, const void* w, int
   return PE_OK;
 }
 
-// The prefill's NF4 linears: all M rows (A-tiled) in blocks of 256 rows on
-// grid.z, one K split, each weight dequantised once per row block. SwiGLU
-// (out_units > 0, bf16): the activation stored A-tiled; otherwise fp32 sums
-// y[M][N] (one split of partials).
-int pe_internal_nf4_prefill(const void* x_tiled, int M, int K, const void* w, const void* wabs, int N, float* y,
-                            void* act, int out_units, hipStream_t st) {
-  if (!x_tiled || !w || !wabs || M <= 0 || K % 128 || N % (32 * kBigNT)) return PE_ERR_ARG;
-  if (out_units ? (!act || out_units * 128 != N / 2) : !y) return PE_ERR_ARG;
-  const int units = K / 128, groups = N / (32 * kBigNT), mtiles = (M + 31) / 32;
-  const dim3 grid(groups, 1, (mtiles + 7) / 8);
-  if (out_units) {
-    EpiArgs e = make_epi(PE_EPI_SWIGLU, M, N, nullptr, nullptr, 0, act, 0);
-    e.out_units = out_units;
-    nf4_gemm_bigws_kernel<true><<<grid, kWsWaves * 64, 0, st>>>((const uint16_t*)x_tiled, (const uint8_t*)w,
-                                                                (const uint16_t*)wabs, units, units, mtiles, e);
-  } else {
-    EpiArgs e = make_epi(kEpiPartial, M, N, nullptr, nullptr, 0, y, N);
-    nf4_gemm_bigws_kernel<false><<<grid, kWsWaves * 64, 0, st>>>((const uint16_t*)x_tiled, (const uint8_t*)w,
-                                                                 (const uint16_t*)wabs, units, units, mtiles, e);
-  }
+
+namespace {
+// The many-row NF4 launch of a plan: fp32 partials (act null) or, unsplit, the
+// SwiGLU activation stored A-tiled.
+int launch_bigws(int wfmt, const BigPlan& p, const void* x_tiled, int M, const void* w, const void* wabs,
+                 const EpiArgs& e, hipStream_t st) {
+  const int mtiles = (M + 31) / 32;
+  const dim3 grid(p.groups, p.S, (mtiles + 7) / 8);
+  const bool sw = e.op == PE_EPI_SWIGLU, af = wfmt == PE_WFMT_NF4_F32ABS;
+#define PE_BIGWS(SW, AF)                                                                              \
+  nf4_gemm_bigws_kernel<SW, AF><<<grid, kWsWaves * 64, 0, st>>>((const uint16_t*)x_tiled, (const uint8_t*)w, wabs, \
+                                                                p.units, p.pps, mtiles, e)
+  if (sw && af) PE_BIGWS(true, true);
+  else if (sw) PE_BIGWS(true, false);
+  else if (af) PE_BIGWS(false, true);
+  else PE_BIGWS(false, false);
+#undef PE_BIGWS
   PE_CHECK_LAUNCH();
   return PE_OK;
 }
 
-int pe_internal_nf4_bigm_partials(const void* x_tiled, int M, int K, const void* w, const void* wabs, int N,
-                                  float* partial, int64_t partial_bytes, int* splits, hipStream_t st) {
-  if (!x_tiled || !w || !wabs || !partial || !splits || M <= 0 || M > 8 * 32 || K % 128 || N % (32 * kBigNT))
-    return PE_ERR_ARG;
-  const BigPlan p = big_plan(N, K);
-  if (partial_bytes < (int64_t)p.S * M * N * 4) return PE_ERR_WORKSPACE;
-  EpiArgs e = make_epi(kEpiPartial, M, N, nullptr, nullptr, 0, partial, N);
+// K splits a dense many-row linear may take: the kernels that sum its partials
+// re-read them all.
+constexpr int kDenseMaxSplits = 8;
+}  // namespace
+
+bool pe_internal_many_fits(int N, int K) { return N > 0 && K >= 128 && N % (32 * kBigNT) == 0 && K % 128 == 0; }
+
+int64_t pe_internal_many_partials_bytes(int wfmt, int M, int N, int K) {
+  if (M <= 0 || !pe_internal_many_fits(N, K)) return 0;
+  const int S = pe_wfmt_nf4(wfmt) ? big_plan(M, N, K).S : dense_bigm_splits(M, N, K, kDenseMaxSplits);
+  return (int64_t)S * M * N * 4;
+}
+
+int pe_internal_many_linear(int wfmt, int dtype, const void* x_tiled, int M, int K, const void* w, const void* wabs,
+                            int N, float* partial, int64_t partial_bytes, int* splits, hipStream_t st) {
+  if (!x_tiled || !w || !partial || !splits || M <= 0 || !pe_internal_many_fits(N, K)) return PE_ERR_ARG;
+  if (partial_bytes < pe_internal_many_partials_bytes(wfmt, M, N, K)) return PE_ERR_WORKSPACE;
+  if (!pe_wfmt_nf4(wfmt))
+    return pe_internal_dense_bigm(x_tiled, M, K, w, dtype, N, partial, N, st, true, splits, kDenseMaxSplits);
+  if (!wabs) return PE_ERR_ARG;
+  const BigPlan p = big_plan(M, N, K);
   *splits = p.S;
-  const int mtiles = (M + 31) / 32;
-  nf4_gemm_bigws_kernel<false><<<dim3(p.groups, p.S), kWsWaves * 64, 0, st>>>(
-      (const uint16_t*)x_tiled, (const uint8_t*)w, (const uint16_t*)wabs, p.units, p.pps, mtiles, e);
-  PE_CHECK_LAUNCH();
-  return PE_OK;
+  return launch_bigws(wfmt, p, x_tiled, M, w, wabs, make_epi(kEpiPartial, M, N, nullptr, nullptr, 0, partial, N), st);
 }
 
-int pe_internal_nf4_bigm_swiglu(const void* x_tiled, int M, int K, const void* w, const void* wabs, int N, void* out,
-                                int out_units, int dtype, float* partial, int64_t partial_bytes, int* splits,
-                                hipStream_t st) {
-  if (!x_tiled || !w || !wabs || !out || !splits || M <= 0 || M > 8 * 32 || K % 128 || N % (32 * kBigNT) ||
-      out_units * 128 != N / 2)
+int pe_internal_many_swiglu(int wfmt, int dtype, const void* x_tiled, int M, int K, const void* w, const void* wabs,
+                            int N, void* out, int out_units, float* partial, int64_t partial_bytes, int* splits,
+                            hipStream_t st) {
+  if (!x_tiled || !w || !out || !splits || M <= 0 || !pe_internal_many_fits(N, K) || out_units * 256 != N)
     return PE_ERR_ARG;
-  const BigPlan p = big_plan(N, K);
-  if (p.S > 1 || dtype != PE_DTYPE_BF16)
-    return pe_internal_nf4_bigm_partials(x_tiled, M, K, w, wabs, N, partial, partial_bytes, splits, st);
-  EpiArgs e = make_epi(PE_EPI_SWIGLU, M, N, nullptr, nullptr, 0, out, 0);
-  e.out_units = out_units;
   *splits = 0;
-  const int mtiles = (M + 31) / 32;
-  nf4_gemm_bigws_kernel<true><<<dim3(p.groups, 1), kWsWaves * 64, 0, st>>>(
-      (const uint16_t*)x_tiled, (const uint8_t*)w, (const uint16_t*)wabs, p.units, p.pps, mtiles, e);
-  PE_CHECK_LAUNCH();
-  return PE_OK;
+  if (!pe_wfmt_nf4(wfmt)) {
+    if (t256_shape(M, N, K))
+      return t256_launch(x_tiled, M, K, w, dtype, N, out, 0, kEpiTSwiglu, out_units, t256_plan(M, N, K, 1, false), st);
+  } else {
+    if (!wabs) return PE_ERR_ARG;
+    const BigPlan p = big_plan(M, N, K);
+    if (p.S == 1 && dtype == PE_DTYPE_BF16) {
+      EpiArgs e = make_epi(PE_EPI_SWIGLU, M, N, nullptr, nullptr, 0, out, 0);
+      e.out_units = out_units;
+      return launch_bigws(wfmt, p, x_tiled, M, w, wabs, e, st);
+    }
+  }
+  return pe_internal_many_linear(wfmt, dtype, x_tiled, M, K, w, wabs, N, partial, partial_bytes, splits, st);
 }
 
-// A dense 16-bit pe_dense_gemm of more than 256 rows without bias or residual
+// A dense 16-bit pe_dense_gemm of more than 64 rows without bias or residual
 // packs X A-tiled into its workspace and runs the many-row kernel.
 static bool dense_many_rows(int M, int N, int K, int epilogue, const void* bias) {
-  return M > 4 * kMaxChunkRows && epilogue == PE_EPI_STORE && !bias && K % 128 == 0 && N % (32 * kBigNT) == 0;
+  return M > kMaxChunkRows && epilogue == PE_EPI_STORE && !bias && K % 128 == 0 && N % (32 * kBigNT) == 0;
 }
 
 extern "C" int64_t pe_gemm_workspace_bytes(int M, int N, int K, int wfmt, int dtype, int epilogue) {
@@ -2185,7 +2185,7 @@ extern "C" int64_t pe_gemm_workspace_bytes(int M, int N, int K, int wfmt, int dt
   // of pe_nf4_gemm_tiled needs its split partials when its plan splits K
   const bool nf4 = pe_wfmt_nf4(wfmt);
   const int64_t big = nf4 && epilogue == PE_EPI_SWIGLU && M > kMaxChunkRows && M <= 8 * 32
-                          ? pe_internal_nf4_bigm_partials_bytes(M, N, K)
+                          ? pe_internal_many_partials_bytes(wfmt, M, N, K)
                           : 0;
   const int mc = M > kMaxChunkRows ? kMaxChunkRows : M;
   int64_t w = workspace_of(make_plan(mc, N, K, nf4, epilogue));
@@ -2225,8 +2225,8 @@ extern "C" int pe_nf4_gemm_tiled(const void* x_tiled, int M, int K, const uint8_
     if (M > 8 * 32 || epilogue != PE_EPI_SWIGLU || bias || out_units * 256 != N) return PE_ERR_ARG;
     int S = 0;
     const hipStream_t st = (hipStream_t)stream;
-    int rc = pe_internal_nf4_bigm_swiglu(x_tiled, M, K, w_tiled, absmax_tiled, N, out, out_units, PE_DTYPE_BF16,
-                                         (float*)workspace, workspace_bytes, &S, st);
+    int rc = pe_internal_many_swiglu(PE_WFMT_NF4, PE_DTYPE_BF16, x_tiled, M, K, w_tiled, absmax_tiled, N, out,
+                                     out_units, (float*)workspace, workspace_bytes, &S, st);
     if (rc == PE_OK && S > 0)
       rc = pe_internal_swiglu_partials((const float*)workspace, S, M, N, out, ld_out, out_units, PE_DTYPE_BF16, st);
     return rc;
@@ -2236,7 +2236,7 @@ extern "C" int pe_nf4_gemm_tiled(const void* x_tiled, int M, int K, const uint8_
 }
 
 extern "C" int64_t pe_nf4_gemm_partials_bytes(int M, int N, int K) {
-  if (M > kMaxChunkRows && M <= 8 * 32) return pe_internal_nf4_bigm_partials_bytes(M, N, K);
+  if (M > kMaxChunkRows && M <= 8 * 32) return pe_internal_many_partials_bytes(PE_WFMT_NF4, M, N, K);
   if (M <= 0 || M > kMaxChunkRows || N <= 0 || K < 128) return 0;
   return pe_internal_linear_partials_bytes(M, N, K, PE_WFMT_NF4);
 }
@@ -2246,8 +2246,9 @@ extern "C" int pe_nf4_gemm_partials(const void* x, int64_t ldx, int x_tiled, int
                                     int* splits, void* stream) {
   if (M > kMaxChunkRows) {  // the many-row kernel: A-tiled X, N % 128 == 0
     if (!x_tiled) return PE_ERR_ARG;
-    return pe_internal_nf4_bigm_partials(x, M, K, w_tiled, absmax_tiled, N, partials, partial_bytes, splits,
-                                         (hipStream_t)stream);
+    if (M > 8 * 32) return PE_ERR_ARG;
+    return pe_internal_many_linear(PE_WFMT_NF4, PE_DTYPE_BF16, x, M, K, w_tiled, absmax_tiled, N, partials,
+                                   partial_bytes, splits, (hipStream_t)stream);
   }
   return pe_internal_linear_partials(PE_WFMT_NF4, PE_DTYPE_BF16, x, x_tiled ? K : ldx, x_tiled != 0, M, K, w_tiled,
                                      absmax_tiled, N, partials, partial_bytes, splits, (hipStream_t)stream);
@@ -2297,7 +2298,8 @@ extern "C" int pe_dense_gemm(const void* x, int64_t ldx, int M, int K, const voi
   if (dtype != PE_DTYPE_BF16 && dtype != PE_DTYPE_F16) return PE_ERR_ARG;
   if (dense_many_rows(M, N, K, epilogue, bias) && workspace && workspace_bytes >= kCounterBytes + xtile_bytes(M, K)) {
     // every weight read once per 256 rows instead of once per 64-row launch;
-    // the A-tiled rows after the workspace's counters
+    // the A-tiled rows after the workspace's counters (a smaller workspace
+    // keeps the 64-row launches)
     if (!x || !w || !out || ld_out < N || ldx < K) return PE_ERR_ARG;
     void* xt = (char*)workspace + kCounterBytes;
     int rc = pe_internal_to_xtile(x, ldx, M, K, xt, st);

@@ -57,35 +57,29 @@ PE_INTERNAL int pe_internal_rope_kv_partials(const float* partial, int S, int M,
 // MFMA-tiled layout, K % 128 == 0, N % 128 == 0), each weight read once per
 // block of up to 256 rows; Y row-major (leading dimension ld_out) in the
 // dtype, or the fp32 sums as they are (f32_out: split partials
-// [S][M][ld_out] for the prefill's epilogue kernels; with `splits` given the
-// launch takes up to max_splits K splits and reports S there, else S = 1).
+// [S][M][ld_out]; with `splits` given the launch takes up to max_splits K
+// splits and reports S there, else S = 1).
 PE_INTERNAL int pe_internal_dense_bigm(const void* x_tiled, int M, int K, const void* w, int dtype, int N, void* out,
                                        int64_t ld_out, hipStream_t st, bool f32_out = false,
                                        int* splits = nullptr, int max_splits = 1);
-// The dense gate/up linear over many rows (N = 256 * out_units interleaved
-// columns) storing the SwiGLU activation A-tiled; shapes that fit only.
-PE_INTERNAL bool pe_internal_dense_swiglu_fits(int M, int N, int K);
-PE_INTERNAL int pe_internal_dense_swiglu(const void* x_tiled, int M, int K, const void* w, int dtype, int N, void* act,
-                                         int out_units, hipStream_t st);
-// The prefill's NF4 linear over all M rows (A-tiled X, blocks of 256 rows, one
-// K split): fp32 sums y[M][N], or with out_units > 0 (the interleaved gate/up
-// weight, N = 2 * 128 * out_units) the SwiGLU activation stored A-tiled.
-PE_INTERNAL int pe_internal_nf4_prefill(const void* x_tiled, int M, int K, const void* w, const void* wabs, int N,
-                                        float* y, void* act, int out_units, hipStream_t st);
+// A pass's linear over many rows (more than 64, A-tiled X; pe_internal_many_fits
+// shapes) in any 16-bit weight format (PE_WFMT_*): fp32 split partials
+// [S][M][N], *splits receives S. NF4 weights are dequantised once per block of
+// 256 rows.
+PE_INTERNAL bool pe_internal_many_fits(int N, int K);
+PE_INTERNAL int64_t pe_internal_many_partials_bytes(int wfmt, int M, int N, int K);
+PE_INTERNAL int pe_internal_many_linear(int wfmt, int dtype, const void* x_tiled, int M, int K, const void* w,
+                                        const void* wabs, int N, float* partial, int64_t partial_bytes, int* splits,
+                                        hipStream_t st);
+// The same with the SwiGLU of an interleaved gate/up weight (N = 256 *
+// out_units): the GEMM stores the A-tiled activation itself and *splits = 0,
+// or it writes split partials (*splits = S) for pe_internal_swiglu_partials.
+PE_INTERNAL int pe_internal_many_swiglu(int wfmt, int dtype, const void* x_tiled, int M, int K, const void* w,
+                                        const void* wabs, int N, void* out, int out_units, float* partial,
+                                        int64_t partial_bytes, int* splits, hipStream_t st);
 // Row-major 16-bit [M][K] (leading dimension ld) -> the A-tiled layout
 // (K % 128 == 0; rows past M of the last 32-row tile are written as zeros).
 PE_INTERNAL int pe_internal_to_xtile(const void* x, int64_t ld, int M, int K, void* out, hipStream_t st);
-PE_INTERNAL int64_t pe_internal_nf4_bigm_partials_bytes(int M, int N, int K);
-PE_INTERNAL int pe_internal_nf4_bigm_partials(const void* x_tiled, int M, int K, const void* w, const void* wabs,
-                                              int N, float* partial, int64_t partial_bytes, int* splits,
-                                              hipStream_t st);
-// The gate/up linear of the many-row pass with its SwiGLU: when the plan has
-// one split (and bf16 compute) the GEMM stores the A-tiled activation itself
-// and *splits = 0; otherwise it writes split partials (*splits = S) for
-// pe_internal_swiglu_partials.
-PE_INTERNAL int pe_internal_nf4_bigm_swiglu(const void* x_tiled, int M, int K, const void* w, const void* wabs, int N,
-                                            void* out, int out_units, int dtype, float* partial, int64_t partial_bytes,
-                                            int* splits, hipStream_t st);
 PE_INTERNAL int pe_internal_swiglu_partials(const float* partial, int S, int M, int N, void* out, int64_t ld_out,
                                             int out_units, int dtype, hipStream_t st);
 

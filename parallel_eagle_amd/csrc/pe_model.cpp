@@ -162,20 +162,20 @@ extern "C" int pe_version(void) { return 1; }
 constexpr int kFusedChunk = 64;  // rows per fused pass (causal passes are chunked)
 
 // ---------------------------------------------------------------------------
-// Prefill (a causal pass of more than 256 rows of a 16-bit model, NF4 or
-// dense, with RoPE-paired q/k/v and 128-dim heads): every linear runs once
-// over all M rows in blocks of 256 rows on the matrix cores
-// (pe_internal_nf4_prefill: each NF4 weight dequantised once per row block by
-// producer waves; pe_internal_dense_bigm: 16-bit tiled weights), with the
-// activations A-tiled between kernels. The GEMMs write fp32 sums that the
-// fused pass's epilogue kernels treat as one split: RoPE + K/V append for
-// q/k/v, SwiGLU for a dense gate/up (the NF4 gate/up stores the activation
-// itself), residual + RMSNorm (with the captures) after o and down.
-// Attention runs once over all rows, causally. NF4 weights with fp32 absmax
-// (checkpoint imports) are dequantised and tiled to 16-bit once per linear
-// and prefill. Shorter causal passes run as 64-row chunks of the fused pass.
+// Prefill (a causal pass of more than one fused chunk of a 16-bit model, NF4
+// or dense, with RoPE-paired q/k/v and 128-dim heads): every linear runs once
+// over all M rows on the matrix cores (pe_internal_many_linear: each NF4
+// weight dequantised once per block of 256 rows by producer waves, or 16-bit
+// tiled weights), with the activations A-tiled between kernels. The GEMMs
+// write fp32 split partials for the fused pass's epilogue kernels: RoPE + K/V
+// append for q/k/v, residual + RMSNorm (with the captures) after o and down;
+// gate/up stores the SwiGLU activation itself where it runs unsplit.
+// Attention runs once over all rows, causally. (150 rows at the 7B width over
+// 900 cached ones, four layers of fp32-absmax weights: 1346 us as three
+// 64-row chunks of the fused pass, each of which streams and dequantises every
+// weight.)
 // ---------------------------------------------------------------------------
-constexpr int kPrefillMinRows = 4 * kFusedChunk + 1;
+constexpr int kPrefillMinRows = kFusedChunk + 1;
 bool prefill_path(const pe_model_desc* m, int M, int mask_mode) {
   static const bool on = [] {
     const char* v = getenv("PE_PREFILL_GEMM");
@@ -188,14 +188,22 @@ bool prefill_path(const pe_model_desc* m, int M, int mask_mode) {
          ((m->num_heads + 2 * m->num_kv_heads) * m->head_dim) % 128 == 0 && m->vocab % 128 == 0;
 }
 
+// fp32 split partials of a layer's widest many-row linear.
+int64_t many_partials_bytes(const pe_model_desc* m, int M) {
+  const int H = m->hidden, qd = m->num_heads * m->head_dim, ip = m->intermediate_padded;
+  const int nqkv = qd + 2 * m->num_kv_heads * m->head_dim, wf = m->weight_format;
+  return std::max(std::max(pe_internal_many_partials_bytes(wf, M, nqkv, H), pe_internal_many_partials_bytes(wf, M, H, qd)),
+                  std::max(pe_internal_many_partials_bytes(wf, M, 2 * ip, H), pe_internal_many_partials_bytes(wf, M, H, ip)));
+}
+
 struct PrefillLayout {
-  int64_t h, xn, xn_t, q, attn, attn_t, act_t, y, ny, wdeq, wtile, attn_ws, attn_ws_bytes, gemm, gemm_bytes, total;
+  int64_t h, xn_t, q, attn, attn_t, act_t, y, y_bytes, attn_ws, attn_ws_bytes, gemm, gemm_bytes, total;
 };
 
 PrefillLayout make_prefill_layout(const pe_model_desc* m, int M, int64_t kv_len) {
   PrefillLayout L;
   const int64_t H = m->hidden, qd = (int64_t)m->num_heads * m->head_dim;
-  const int64_t nqkv = qd + 2ll * m->num_kv_heads * m->head_dim, ip = m->intermediate_padded;
+  const int64_t ip = m->intermediate_padded;
   // offset 0: the pass's arrival counters, as in the fused layout (the GEMM
   // and attention counter slices rest at zero between passes, whichever path
   // ran last)
@@ -208,26 +216,13 @@ PrefillLayout make_prefill_layout(const pe_model_desc* m, int M, int64_t kv_len)
     return o;
   };
   L.h = take(M * H * 2);
-  L.xn = take(M * H * 2);
   L.xn_t = take(xtile_bytes(M, (int)H));
   L.q = take(M * qd * 2);
   L.attn = take(M * qd * 2);
   L.attn_t = take(xtile_bytes(M, (int)qd));
   L.act_t = take(xtile_bytes(M, (int)ip));
-  int64_t ny = nqkv;
-  if (2 * ip > ny) ny = 2 * ip;
-  if (H > ny) ny = H;
-  L.ny = 2 * ny;  // fp32 partials: up to four K splits of the narrower linears, two of the widest
-  L.y = take(M * L.ny * 4);
-  L.wdeq = L.wtile = 0;
-  if (m->weight_format == PE_WFMT_NF4_F32ABS) {  // one linear dequantised, then tiled
-    int64_t nw = nqkv * H;
-    if (2 * ip * H > nw) nw = 2 * ip * H;
-    if (H * ip > nw) nw = H * ip;
-    if (H * qd > nw) nw = H * qd;
-    L.wdeq = take(nw * 2);
-    L.wtile = take(nw * 2);
-  }
+  L.y_bytes = many_partials_bytes(m, M);
+  L.y = take(L.y_bytes);
   L.attn_ws_bytes = align_up(attention_workspace_bytes(M, m->num_heads, m->num_kv_heads, m->head_dim, kv_len,
                                                        m->dtype, m->attn_mode));
   L.attn_ws = take(L.attn_ws_bytes);
@@ -259,7 +254,6 @@ int forward_prefill(const pe_model_desc* m, const pe_pass_args* a, const Prefill
   const int qd = nh * hd, ip = m->intermediate_padded, L = m->num_layers;
   const int nqkv = (nh + 2 * nkv) * hd;
   void* h = ws + Lp.h;
-  void* xn = ws + Lp.xn;
   void* xn_t = ws + Lp.xn_t;
   void* q = ws + Lp.q;
   void* attn = ws + Lp.attn;
@@ -269,7 +263,6 @@ int forward_prefill(const pe_model_desc* m, const pe_pass_args* a, const Prefill
   const float scale = (float)(1.0 / std::sqrt((double)hd));
   const int64_t layer_stride = (int64_t)nkv * a->cache_capacity * hd * es;
   const int64_t fused_ld = (int64_t)a->num_features * H;
-  const bool nf4 = m->weight_format == PE_WFMT_NF4;
   int rc;
 #define PE_TRY(expr)            \
   do {                          \
@@ -292,25 +285,11 @@ int forward_prefill(const pe_model_desc* m, const pe_pass_args* a, const Prefill
     }
     return PE_OK;
   };
-  // a dense weight as stored, or fp32-absmax NF4 codes dequantised and tiled to 16 bits
-  auto dense_weight = [&](const void* w, const void* ab, int N, int K, const void** wt) -> int {
-    *wt = w;
-    if (m->weight_format != PE_WFMT_NF4_F32ABS) return PE_OK;
-    int r = pe_nf4_dequant_f32abs((const uint8_t*)w, (const float*)ab, N, K, (uint16_t*)(ws + Lp.wdeq), st);
-    if (r != PE_OK) return r;
-    *wt = ws + Lp.wtile;
-    return pe_dense_repack(ws + Lp.wdeq, N, K, m->dtype, ws + Lp.wtile, st);
-  };
   // y[ys][M][N] (fp32 split partials) = x (A-tiled) . W^T over all rows
-  int ys = 1;
+  const int wf = m->weight_format;
+  int ys = 0;
   auto linear = [&](const void* xt, int K, const void* w, const void* ab, int N) -> int {
-    ys = 1;
-    if (nf4) return pe_internal_nf4_prefill(xt, M, K, w, ab, N, y, nullptr, 0, st);
-    const void* wt;
-    const int r = dense_weight(w, ab, N, K, &wt);
-    if (r != PE_OK) return r;
-    const int most = (int)std::min<int64_t>(4, Lp.ny / N);
-    return pe_internal_dense_bigm(xt, M, K, wt, m->dtype, N, y, N, st, true, &ys, most);
+    return pe_internal_many_linear(wf, m->dtype, xt, M, K, w, ab, N, y, Lp.y_bytes, &ys, st);
   };
 
   {
@@ -336,16 +315,9 @@ int forward_prefill(const pe_model_desc* m, const pe_pass_args* a, const Prefill
     PE_TRY(linear(attn_t, qd, m->w_o[l], m->a_o ? m->a_o[l] : nullptr, H));
     PE_TRY(pe_internal_residual_rmsnorm(y, ys, M, h, H, m->mlp_norm[l], m->rms_eps, m->norm_mode, m->dtype, nullptr, xn_t,
                                         nullptr, 0, nullptr, 0, st));
-    if (nf4) {
-      PE_TRY(pe_internal_nf4_prefill(xn_t, M, H, m->w_gu[l], m->a_gu[l], 2 * ip, nullptr, act_t, ip / 128, st));
-    } else if (pe_internal_dense_swiglu_fits(M, 2 * ip, H)) {
-      const void* wt;
-      PE_TRY(dense_weight(m->w_gu[l], m->a_gu ? m->a_gu[l] : nullptr, 2 * ip, H, &wt));
-      PE_TRY(pe_internal_dense_swiglu(xn_t, M, H, wt, m->dtype, 2 * ip, act_t, ip / 128, st));
-    } else {
-      PE_TRY(linear(xn_t, H, m->w_gu[l], m->a_gu ? m->a_gu[l] : nullptr, 2 * ip));
-      PE_TRY(pe_internal_swiglu_partials(y, ys, M, 2 * ip, act_t, ip, ip / 128, m->dtype, st));
-    }
+    PE_TRY(pe_internal_many_swiglu(wf, m->dtype, xn_t, M, H, m->w_gu[l], m->a_gu ? m->a_gu[l] : nullptr, 2 * ip, act_t,
+                                   ip / 128, y, Lp.y_bytes, &ys, st));
+    if (ys > 0) PE_TRY(pe_internal_swiglu_partials(y, ys, M, 2 * ip, act_t, ip, ip / 128, m->dtype, st));
     PE_TRY(linear(act_t, ip, m->w_down[l], m->a_down ? m->a_down[l] : nullptr, H));
     const bool last = l + 1 == L;
     const int fh = last ? -1 : slot_of(l + 1);
@@ -524,14 +496,14 @@ struct BatchLayout {
   int64_t total;
 };
 
-// The batched NF4 pass over 65..256 rows dequantises each weight once for all
-// rows (pe_internal_nf4_bigm_partials) and hands A-tiled activations between
-// the kernels; other batches run each linear in 64-row launches on row-major X.
+// The batched pass over more than 64 rows runs each linear once over all rows
+// (pe_internal_many_linear) and hands A-tiled activations between the kernels;
+// smaller batches run each linear in one launch on row-major X.
 bool batch_big_path(const pe_model_desc* m, int M) {
   const int H = m->hidden, qd = m->num_heads * m->head_dim, ip = m->intermediate_padded;
   const int nqkv = qd + 2 * m->num_kv_heads * m->head_dim;
-  return m->weight_format == PE_WFMT_NF4 && M > kFusedChunk && M <= 256 && H % 128 == 0 && qd % 128 == 0 &&
-         ip % 128 == 0 && nqkv % 128 == 0;
+  return M > kFusedChunk && m->dtype != PE_DTYPE_F32 && H % 128 == 0 && qd % 128 == 0 && ip % 128 == 0 &&
+         nqkv % 128 == 0;
 }
 
 BatchLayout make_batch_layout(const pe_model_desc* m, int M, int max_rows, int64_t max_kv_len, int batch) {
@@ -569,11 +541,7 @@ BatchLayout make_batch_layout(const pe_model_desc* m, int M, int max_rows, int64
     L.xn_t = take(xtile_bytes(M, H));
     L.attn_t = take(xtile_bytes(M, qd));
     L.act_t = take(xtile_bytes(M, ip));
-    const int64_t pb[4] = {pe_internal_nf4_bigm_partials_bytes(M, nqkv, H), pe_internal_nf4_bigm_partials_bytes(M, H, qd),
-                           pe_internal_nf4_bigm_partials_bytes(M, 2 * ip, H), pe_internal_nf4_bigm_partials_bytes(M, H, ip)};
-    for (int i = 0; i < 4; ++i)
-      if (pb[i] > L.part_bytes) L.part_bytes = pb[i];
-    L.part_bytes = align_up(L.part_bytes);
+    L.part_bytes = align_up(many_partials_bytes(m, M));
     L.part = take(L.part_bytes);
   }
   L.total = off;
@@ -646,7 +614,8 @@ int forward_batched(const pe_model_desc* m, const pe_pass_args* a, const BatchLa
     for (int l = 0; l < L; ++l) {
       char* kc = (char*)a->k_cache + l * layer_stride;
       char* vc = (char*)a->v_cache + l * layer_stride;
-      PE_TRY(pe_internal_nf4_bigm_partials(xn_t, M, H, m->w_qkv[l], m->a_qkv[l], nqkv, part, Lb.part_bytes, &S, st));
+      PE_TRY(pe_internal_many_linear(wf, m->dtype, xn_t, M, H, m->w_qkv[l], m->a_qkv ? m->a_qkv[l] : nullptr, nqkv, part,
+                                     Lb.part_bytes, &S, st));
       PE_TRY(pe_internal_rope_kv_partials(part, S, M, nh, nkv, hd, m->b_qkv ? m->b_qkv[l] : nullptr, a->positions,
                                           m->rope_cos_sin, m->max_positions, q, kc, vc, a->cache_capacity, 0,
                                           a->status, m->dtype, st, kvoff));
@@ -654,13 +623,15 @@ int forward_batched(const pe_model_desc* m, const pe_pass_args* a, const BatchLa
                                               a->max_seq_rows, a->prefix_len, a->batch, a->seq_row0, a->seq_prefix,
                                               a->tree_bits, a->bits_words, scale, m->dtype, attn_t, qd, qd / 128,
                                               ws + Lb.attn_ws, Lb.attn_ws_bytes, (int*)gws + kPassAttnCounterInt, st));
-      PE_TRY(pe_internal_nf4_bigm_partials(attn_t, M, qd, m->w_o[l], m->a_o[l], H, part, Lb.part_bytes, &S, st));
+      PE_TRY(pe_internal_many_linear(wf, m->dtype, attn_t, M, qd, m->w_o[l], m->a_o ? m->a_o[l] : nullptr, H, part,
+                                     Lb.part_bytes, &S, st));
       PE_TRY(pe_internal_residual_rmsnorm(part, S, M, h, H, m->mlp_norm[l], m->rms_eps, m->norm_mode, m->dtype, xn,
                                           xn_t, nullptr, 0, nullptr, 0, st));
-      PE_TRY(pe_internal_nf4_bigm_swiglu(xn_t, M, H, m->w_gu[l], m->a_gu[l], 2 * ip, act_t, ip / 128, m->dtype, part,
-                                         Lb.part_bytes, &S, st));
+      PE_TRY(pe_internal_many_swiglu(wf, m->dtype, xn_t, M, H, m->w_gu[l], m->a_gu ? m->a_gu[l] : nullptr, 2 * ip, act_t,
+                                     ip / 128, part, Lb.part_bytes, &S, st));
       if (S > 0) PE_TRY(pe_internal_swiglu_partials(part, S, M, 2 * ip, act_t, ip, ip / 128, m->dtype, st));
-      PE_TRY(pe_internal_nf4_bigm_partials(act_t, M, ip, m->w_down[l], m->a_down[l], H, part, Lb.part_bytes, &S, st));
+      PE_TRY(pe_internal_many_linear(wf, m->dtype, act_t, M, ip, m->w_down[l], m->a_down ? m->a_down[l] : nullptr, H, part,
+                                     Lb.part_bytes, &S, st));
       const bool last = l + 1 == L;
       const int fh = last ? -1 : slot_of(l + 1);
       const int fx = last ? slot_of(L) : -1;
