@@ -56,6 +56,11 @@ __device__ __forceinline__ bool tree_key_allowed(int64_t key, int64_t P, const u
   return (w >> (u & 63)) & 1ull;
 }
 
+// key_allowed with the tree word chosen by selects
+__device__ __forceinline__ bool tree_or_causal(int64_t key, int64_t P, int t, int mask_mode, const uint64_t* nb) {
+  return mask_mode == PE_MASK_CAUSAL ? key <= P + t : tree_key_allowed(key, P, nb);
+}
+
 // One workgroup = 8 waves = one (KV head, key split, 32-row tile); each wave
 // takes a contiguous run of the split's 32-key blocks. Its first two blocks
 // are loaded and processed together as one 64-key block (a run of one block
@@ -1208,6 +1213,87 @@ __global__ __launch_bounds__(128) void attn_generic_kernel(
   }
 }
 
+// fp32 rows of whole 16-byte pieces (hd % 4 == 0, 16-byte aligned): one block per
+// (row t, query head) as above, LPK lanes (at least hd / 4) on one key at a
+// time, so that K and V rows are read whole, 256 / LPK keys in step; the
+// scores stay in LDS up to kF32LdsKeys keys. The lanes of a key add their
+// products of four dims by a butterfly; the key slots' sums of PV are added in
+// slot order. Bound by the latency of a slot's loads (four keys in flight);
+// one thread per key and per dim read K 256 bytes apart per lane and walked V
+// one row at a time.
+constexpr int kF32LdsKeys = 4096;
+
+template <int LPK>
+__global__ __launch_bounds__(256) void attn_f32_kernel(const float* __restrict__ q, const float* __restrict__ kc,
+                                                       const float* __restrict__ vc, int64_t cap, int nh, int nkv,
+                                                       int hd, int T, int64_t P, int mask_mode,
+                                                       const uint64_t* __restrict__ bits, int words, float scale,
+                                                       int eager, float* __restrict__ out, int64_t ld_out,
+                                                       float* __restrict__ scores /* [T*nh][P+T] */) {
+  constexpr int kSlots = 256 / LPK;
+  const int t = blockIdx.x, hq = blockIdx.y, kvh = hq / (nh / nkv);
+  const int64_t S = P + T;
+  const int sl = threadIdx.x / LPK, li = threadIdx.x % LPK;
+  const bool on = 4 * li < hd;
+  __shared__ float s_sc[kF32LdsKeys];
+  __shared__ float s_o[kSlots][4 * LPK];
+  __shared__ float red[4];
+  float* sc = S <= kF32LdsKeys ? s_sc : scores + ((int64_t)t * nh + hq) * S;
+  uint64_t nb[PE_TREE_MAX_WORDS];
+#pragma unroll
+  for (int w = 0; w < PE_TREE_MAX_WORDS; ++w)
+    nb[w] = (mask_mode == PE_MASK_TREE && w < words) ? bits[(int64_t)t * words + w] : 0ull;
+  const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+  const f32x4_t qv = on ? *(const f32x4_t*)(q + ((int64_t)t * nh + hq) * hd + 4 * li) : zero;
+  const float* kh = kc + (int64_t)kvh * cap * hd + 4 * li;
+  const float* vh = vc + (int64_t)kvh * cap * hd + 4 * li;
+  const float sqrt_hd = sqrtf((float)hd);
+  float lmax = kInitMax;
+#pragma unroll 4
+  for (int64_t j = sl; j < S; j += kSlots) {
+    const f32x4_t kv = on ? *(const f32x4_t*)(kh + j * hd) : zero;
+    float d = fmaf(qv[3], kv[3], fmaf(qv[2], kv[2], fmaf(qv[1], kv[1], qv[0] * kv[0])));
+#pragma unroll
+    for (int o = LPK / 2; o > 0; o >>= 1) d += __shfl_xor(d, o, 64);
+    const float v = tree_or_causal(j, P, t, mask_mode, nb) ? (eager ? __fdiv_rn(d, sqrt_hd) : d * scale) : kMaskedScore;
+    if (li == 0) sc[j] = v;
+    lmax = fmaxf(lmax, v);
+  }
+  lmax = wave_max(lmax);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = lmax;
+  __syncthreads();
+  const float M = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+  __syncthreads();
+  float lsum = 0.f;
+  for (int64_t j = threadIdx.x; j < S; j += 256) {
+    const float p = expf(sc[j] - M);
+    sc[j] = p;
+    lsum += p;
+  }
+  lsum = wave_sum(lsum);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = lsum;
+  __syncthreads();
+  const float L = (red[0] + red[1]) + (red[2] + red[3]);
+  const float invL = 1.0f / L;
+  f32x4_t acc = zero;
+#pragma unroll 4
+  for (int64_t j = sl; j < S; j += kSlots) {
+    const float p = sc[j];
+    const f32x4_t v = on ? *(const f32x4_t*)(vh + j * hd) : zero;
+    const float pr = eager ? __fmul_rn(p, invL) : p;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i] = p != 0.f ? fmaf(pr, v[i], acc[i]) : acc[i];
+  }
+  *(f32x4_t*)&s_o[sl][4 * li] = acc;
+  __syncthreads();
+  for (int d = threadIdx.x; d < hd; d += 256) {
+    float o = 0.f;
+#pragma unroll
+    for (int w = 0; w < kSlots; ++w) o += s_o[w][d];
+    out[(int64_t)t * ld_out + (int64_t)hq * hd + d] = eager ? o : o / L;
+  }
+}
+
 // per-pair arrival counters: zero before first use and between launches
 constexpr int64_t kAttnCounterBytes = 4096;
 
@@ -1926,6 +2012,18 @@ int pe_internal_tree_attention(const void* q, const void* k_cache, const void* v
   }
   dim3 grid(T, nh);
   float* scores = (float*)workspace;
+  if (dtype == PE_DTYPE_F32 && hd % 4 == 0 && (((uintptr_t)q | (uintptr_t)k_cache | (uintptr_t)v_cache) & 15) == 0) {
+#define PE_ATTN_F32(LPK)                                                                                          \
+  attn_f32_kernel<LPK><<<grid, 256, 0, st>>>((const float*)q, (const float*)k_cache, (const float*)v_cache, cache_cap, \
+                                             nh, nkv, hd, T, P, mask_mode, bits, words, scale, eager, (float*)out,   \
+                                             ld_out, scores)
+    if (hd <= 64) PE_ATTN_F32(16);
+    else if (hd <= 128) PE_ATTN_F32(32);
+    else PE_ATTN_F32(64);
+#undef PE_ATTN_F32
+    PE_CHECK_LAUNCH();
+    return PE_OK;
+  }
   switch (dtype) {
     case PE_DTYPE_F32:
       attn_generic_kernel<PE_DTYPE_F32><<<grid, 128, 0, st>>>((const float*)q, (const float*)k_cache,

@@ -457,6 +457,8 @@ void launch_norm(int smax, const NormArgs<typename Elem<DT>::T>& a, hipStream_t 
   }
 }
 
+bool pe_internal_norm_fits(int H) { return H > 0 && H % 4 == 0 && H <= 4 * kNormThreads * kNormChunks; }
+
 int pe_internal_residual_rmsnorm(const float* partial, int S, int M, void* h, int H, const void* w, float eps,
                                  int mode, int dtype, void* xn, void* xn_tiled, void* cap_h, int64_t ld_cap_h, void* cap_xn,
                                  int64_t ld_cap_xn, hipStream_t st) {

@@ -87,6 +87,8 @@ PE_INTERNAL int pe_internal_swiglu_partials(const float* partial, int S, int M, 
 // xn = the RMSNorm of h rounded as `mode` (PE_NORM_*), also A-tiled into xn_tiled when
 // given (xn may then be null: the tiled rows only); optional copies of the new
 // h (cap_h) and of xn (cap_xn) into the fused-feature rows.
+// Row widths the fused norm kernels take.
+PE_INTERNAL bool pe_internal_norm_fits(int H);
 PE_INTERNAL int pe_internal_residual_rmsnorm(const float* partial, int S, int M, void* h, int H, const void* w,
                                              float eps, int mode, int dtype, void* xn, void* xn_tiled, void* cap_h,
                                              int64_t ld_cap_h, void* cap_xn, int64_t ld_cap_xn, hipStream_t st);

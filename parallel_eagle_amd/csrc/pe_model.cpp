@@ -818,23 +818,52 @@ extern "C" int pe_forward(const pe_model_desc* m, const pe_pass_args* a, void* s
     if (rc != PE_OK) return rc; \
   } while (0)
 
-  auto capture = [&](int slot_layer, const void* src) -> int {
-    if (!a->fused) return PE_OK;
-    for (int f = 0; f < a->num_features; ++f) {
-      if (a->feature_layers[f] != slot_layer) continue;
-      int r = pe_copy_rows(src, (int64_t)H * es, M, (int64_t)H * es, (char*)a->fused + (int64_t)f * H * es, fused_ld,
-                           st);
+  // first fused-feature slot of `layer` (or -1), copied to the layer's other slots
+  auto slot_of = [&](int layer) -> int {
+    for (int f = 0; a->fused && f < a->num_features; ++f)
+      if (a->feature_layers[f] == layer) return f;
+    return -1;
+  };
+  auto slot_ptr = [&](int f) -> void* { return f < 0 ? nullptr : (char*)a->fused + (int64_t)f * H * es; };
+  auto capture = [&](int layer, const void* src, int64_t ld_src, int from) -> int {
+    for (int f = from; a->fused && f < a->num_features; ++f) {
+      if (a->feature_layers[f] != layer) continue;
+      int r = pe_copy_rows(src, ld_src, M, (int64_t)H * es, slot_ptr(f), fused_ld, st);
       if (r != PE_OK) return r;
     }
     return PE_OK;
   };
+  // The norms gather the embeddings and store the captured hidden states
+  // (widths of whole 16-byte pieces at 16-byte aligned addresses; otherwise
+  // separate launches do).
+  uintptr_t where = (uintptr_t)m->embed | (uintptr_t)m->final_norm | (uintptr_t)a->fused;
+  for (int l = 0; l < m->num_layers; ++l) where |= (uintptr_t)m->attn_norm[l];
+  const bool fused_norms = pe_internal_norm_fits(H) && where % 16 == 0;
+  // x of `layer`'s hidden state h, normed by w into xn; captures h (layer's slots) and, final, xn (slot num_layers)
+  auto norm = [&](int layer, const void* w, int mode, bool final) -> int {
+    const int fh = final ? -1 : slot_of(layer), fx = final ? slot_of(layer) : -1;
+    const int first = final ? fx : fh;
+    if (!fused_norms) {
+      int r = final ? PE_OK : capture(layer, h, (int64_t)H * es, 0);
+      if (r == PE_OK) r = pe_rmsnorm_ex(h, H, M, H, w, m->rms_eps, m->dtype, mode, xn, H, st);
+      if (r == PE_OK && final) r = capture(layer, xn, (int64_t)H * es, 0);
+      return r;
+    }
+    int r;
+    if (layer == 0 && !final)
+      r = pe_internal_embed_rmsnorm(a->input_ids, M, m->embed, embed_rows(m), h, H, w, m->rms_eps, mode, m->dtype, xn,
+                                    nullptr, slot_ptr(fh), fused_ld / es, nullptr, 0, a->status, st);
+    else
+      r = pe_internal_residual_rmsnorm(nullptr, 0, M, h, H, w, m->rms_eps, mode, m->dtype, xn, nullptr, slot_ptr(fh),
+                                       fused_ld / es, slot_ptr(fx), fused_ld / es, st);
+    return r == PE_OK && first >= 0 ? capture(layer, slot_ptr(first), fused_ld, first + 1) : r;
+  };
 
-  PE_TRY(pe_embed(a->input_ids, M, m->embed, embed_rows(m), H, m->dtype, h, H, a->status, st));
-  PE_TRY(capture(0, h));
+  if (!fused_norms) PE_TRY(pe_embed(a->input_ids, M, m->embed, embed_rows(m), H, m->dtype, h, H, a->status, st));
   for (int l = 0; l < m->num_layers; ++l) {
     void* kc = (char*)a->k_cache + l * layer_stride;
     void* vc = (char*)a->v_cache + l * layer_stride;
-    PE_TRY(pe_rmsnorm_ex(h, H, M, H, m->attn_norm[l], m->rms_eps, m->dtype, m->norm_mode, xn, H, st));
+    PE_TRY(norm(l, m->attn_norm[l], m->norm_mode, false));
     PE_TRY(linear(m, xn, H, M, H, m->w_qkv[l], m->a_qkv ? m->a_qkv[l] : nullptr, nqkv, PE_EPI_STORE,
                   m->b_qkv ? m->b_qkv[l] : nullptr, nullptr, 0, qkv, nqkv, gws, gwsb, st));
     PE_TRY(pe_rope_qkv(qkv, nqkv, M, nh, nkv, hd, a->positions, m->rope_cos_sin, m->max_positions, m->dtype, q, kc, vc,
@@ -849,10 +878,8 @@ extern "C" int pe_forward(const pe_model_desc* m, const pe_pass_args* a, void* s
                   nullptr, 0, act, ip, gws, gwsb, st));
     PE_TRY(linear(m, act, ip, M, ip, m->w_down[l], m->a_down ? m->a_down[l] : nullptr, H, PE_EPI_RESIDUAL, nullptr,
                   h, H, h, H, gws, gwsb, st));
-    if (l + 1 < m->num_layers) PE_TRY(capture(l + 1, h));
   }
-  PE_TRY(pe_rmsnorm(h, H, M, H, m->final_norm, m->rms_eps, m->dtype, xn, H, st));
-  PE_TRY(capture(m->num_layers, xn));
+  PE_TRY(norm(m->num_layers, m->final_norm, PE_NORM_HF, true));
   if (a->logits) PE_TRY(lm_head(m, a, xn, false, M, gws, gwsb, st));
 #undef PE_TRY
   return PE_OK;
