@@ -875,6 +875,33 @@ __global__ __launch_bounds__(64 * kPairWaves, 1) void attn_pair_kernel(
     body(std::false_type());
 }
 
+// Arithmetic of the eager softmax. The masked score is finite (kEagerMasked):
+// exponentials of differences then need no special case.
+constexpr float kEagerMasked = -1.0e30f;
+
+// round(x / sqrt(128)) for x a value of the 16-bit type, the quotient in fp32
+// first (torch divides in fp32). The product with the reciprocal rounds to the
+// same bf16 for every bf16 value; fp16 needs the remainder's correction, which
+// gives the fp32 quotient itself (both checked for all 65536 values; only the
+// sign of a zero may differ).
+template <int DT>
+__device__ __forceinline__ float eager_scaled(float x) {
+  constexpr float kSqrt = 11.3137085f, kInv = 1.0f / kSqrt;
+  float q = x * kInv;
+  if constexpr (DT == PE_DTYPE_F16) q = fmaf(fmaf(-q, kSqrt, x), kInv, q);
+  return Elem<DT>::round(q);
+}
+
+// exp(x) for x <= 0 (finite): 2^(x log2 e), the product's rounding error put
+// back to first order, so that the result is as exact as v_exp_f32
+__device__ __forceinline__ float exp_neg(float x) {
+  constexpr float kHi = 1.44269502162933349609375f, kLo = 1.92596299112661746887e-8f, kLn2 = 0.693147180559945f;
+  const float t = x * kHi;
+  const float e = fmaf(x, kLo, fmaf(x, kHi, -t));
+  const float p = __builtin_amdgcn_exp2f(t);
+  return fmaf(p * kLn2, e, p);
+}
+
 // Eager attention on the matrix cores (PE_ATTN_EAGER, the drafter's attention,
 // src/pe/nn.py:84-87, 16-bit with hd = 128), one key split, so that a
 // workgroup sees every key of its rows: one workgroup = 8 waves = one (KV head,
@@ -882,7 +909,7 @@ __global__ __launch_bounds__(64 * kPairWaves, 1) void attn_pair_kernel(
 // twice.
 //   Pass 1: S^T = K Q^T on MFMA; each score rounded as the reference rounds it
 //   (the product to the dtype, divided by sqrt(hd), to the dtype again; a
-//   masked key is -inf); the row's max and the fp32 sum of exp(s - max) kept
+//   masked key is very low); the row's max and the fp32 sum of exp(s - max) kept
 //   online; the waves' (max, sum) merged in LDS in wave order.
 //   Pass 2: the same scores again; each probability exp(s - M) / L rounded to
 //   the dtype, as softmax(...).to(q.dtype) leaves it, and multiplied by V on
@@ -966,7 +993,6 @@ __global__ __launch_bounds__(64 * kAttnWaves, 1) void attn_eager_kernel(
   }
   __syncthreads();  // Q staged
 
-  const float sqrt_hd = sqrtf((float)HD);
   // the rounded scores of one block (s[i]: key jb + 8*(i/4) + 4*g + (i%4) of row ln)
   auto scores = [&](int jb, int slot, float (&s)[16]) {
     f32x16_t sc;
@@ -986,7 +1012,7 @@ __global__ __launch_bounds__(64 * kAttnWaves, 1) void attn_eager_kernel(
     for (int i = 0; i < 16; ++i) {
       const int64_t kj = jb + 8 * (i >> 2) + 4 * g + (i & 3);
       const bool ok = kj < j1 && key_allowed(kj, P, t, mask_mode, nbits);
-      s[i] = ok ? E::round(__fdiv_rn(E::round(sc[i]), sqrt_hd)) : -INFINITY;
+      s[i] = ok ? eager_scaled<DT>(E::round(sc[i])) : kEagerMasked;
     }
   };
   constexpr std::integral_constant<int, 0> kK0{};
@@ -999,16 +1025,16 @@ __global__ __launch_bounds__(64 * kAttnWaves, 1) void attn_eager_kernel(
     if constexpr (decltype(next_c)::value) load_k(jb + 32, 1 - KS);
     float s[16];
     scores(jb, KS, s);
-    float bmax = -INFINITY;
+    float bmax = kEagerMasked;
 #pragma unroll
     for (int i = 0; i < 16; ++i) bmax = fmaxf(bmax, s[i]);
     bmax = fmaxf(bmax, __shfl_xor(bmax, 32, 64));
     const float mnew = fmaxf(m, bmax);
     float psum = 0.f;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) psum += expf(s[i] - mnew);
+    for (int i = 0; i < 16; ++i) psum += exp_neg(s[i] - mnew);
     psum += __shfl_xor(psum, 32, 64);
-    l = l * expf(m - mnew) + psum;
+    l = l * exp_neg(m - mnew) + psum;
     m = mnew;
   };
   if (b0 < b1) {
@@ -1035,7 +1061,7 @@ __global__ __launch_bounds__(64 * kAttnWaves, 1) void attn_eager_kernel(
   for (int w = 0; w < kAttnWaves; ++w) M = fmaxf(M, s_ml[w][ln][0]);
   float L = 0.f;
 #pragma unroll
-  for (int w = 0; w < kAttnWaves; ++w) L += s_ml[w][ln][1] * expf(s_ml[w][ln][0] - M);
+  for (int w = 0; w < kAttnWaves; ++w) L += s_ml[w][ln][1] * exp_neg(s_ml[w][ln][0] - M);
   const float invL = 1.0f / L;
 
   // ---- pass 2: O = sum_j round(exp(s_j - M) / L) v_j
@@ -1054,8 +1080,7 @@ __global__ __launch_bounds__(64 * kAttnWaves, 1) void attn_eager_kernel(
     uint32_t pb[8];
 #pragma unroll
     for (int i = 0; i < 16; i += 2) {
-      const float p0 = E::round(expf(s[i] - M) * invL), p1 = E::round(expf(s[i + 1] - M) * invL);
-      pb[i >> 1] = pack2_16<DT>(p0, p1);
+      pb[i >> 1] = pack2_16<DT>(exp_neg(s[i] - M) * invL, exp_neg(s[i + 1] - M) * invL);
     }
 #pragma unroll
     for (int c = 0; c < 8; ++c) *(u32x4_t*)&vs[4 * c + (lane >> 4)][(lane & 15) * 8] = vf[c];
@@ -1628,6 +1653,251 @@ __global__ __launch_bounds__(64 * kRowsWaves, 1) void attn_rows_kernel(
 }
 
 // ---------------------------------------------------------------------------
+// Eager causal attention over many query rows (a drafter's context)
+// ---------------------------------------------------------------------------
+// attn_rows_kernel's blocks, waves, key groups and LDS ring with
+// attn_eager_kernel's arithmetic: a block's keys are walked twice, first K alone
+// (the row's max and sum of the rounded scores; the two key groups' merged
+// through LDS), then K and V (each probability normalised, rounded and
+// multiplied, the groups' sums added). attn_eager_kernel has every 32-row tile
+// read K twice and V once from global memory by itself and spent most of its
+// issue on a correctly rounded division and the library exponential per score:
+// 1499 context rows of a 7B-width drafter took 209 us a layer, now 97 (192
+// workgroups; issue of the two passes' scores and exponentials bounds it).
+constexpr int kRowsMlFloats = 2 * 4 * 32 * 2;
+
+template <int DT>
+__global__ __launch_bounds__(64 * kRowsWaves, 1) void attn_eager_rows_kernel(
+    const uint16_t* __restrict__ q, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc, int64_t cap,
+    int nh, int nkv, int T, int64_t P, int nblk, int npair, void* __restrict__ out, int64_t ld_out, int out_units) {
+  typedef Elem<DT> E;
+  constexpr int HD = 128;
+  __shared__ __align__(1024) uint8_t smem[kRowsSmem + kRowsMlFloats * 4];
+  float* s_ml = (float*)(smem + kRowsSmem);  // [key group][tile][row](max, sum)
+  const int total = nkv * npair;
+  const int b = blockIdx.x;
+  const int w = (total & 7) ? b : (b & 7) * (total >> 3) + (b >> 3);
+  const int kvh = w / npair, pair = w - kvh * npair;
+  const int G = nh / nkv, rows = T * G;
+  const int64_t S = P + T;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, ln = lane & 31, g = lane >> 5;
+  const int tile = wave & 3, kg = wave >> 2;
+  const uint16_t* kh = kc + (int64_t)kvh * cap * HD;
+  const uint16_t* vh = vc + (int64_t)kvh * cap * HD;
+  const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem;
+  // as in attn_rows_kernel: wave w loads from step 2 it + w / 4; with V, its
+  // eight loads are half of K's or of V's rows, K alone gives it 16 K rows
+  const int dsp = wave >> 2, dq = wave & 3;
+  const uint16_t* ksrc = uniform_ptr(kh);
+  const uint16_t* dsrc = uniform_ptr(dq < 2 ? kh : vh);
+  auto issue_kv = [&](int it) {
+    const int64_t kb0 = (int64_t)(2 * it + dsp) * kRowsKeys;
+    const uint32_t dst = __builtin_amdgcn_readfirstlane(lds_base + (2 * (it & 1) + dsp) * kRowsStepBytes +
+                                                        (dq < 2 ? 0 : 16384) + (dq & 1) * 8192);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const int row = 32 * (dq & 1) + 4 * k + (lane >> 4);
+      const uint32_t key = (uint32_t)min(kb0 + row, S - 1);
+      lds_dma16(dsrc, key * (HD * 2) + (((lane & 15) ^ swz_row(row)) << 4), dst + k * 1024);
+    }
+  };
+  auto issue_k = [&](int it) {
+    const int64_t kb0 = (int64_t)(2 * it + dsp) * kRowsKeys;
+    const uint32_t dst = __builtin_amdgcn_readfirstlane(lds_base + (2 * (it & 1) + dsp) * kRowsStepBytes + dq * 4096);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int row = 16 * dq + 4 * k + (lane >> 4);
+      const uint32_t key = (uint32_t)min(kb0 + row, S - 1);
+      lds_dma16(ksrc, key * (HD * 2) + (((lane & 15) ^ swz_row(row)) << 4), dst + k * 1024);
+    }
+  };
+
+  for (int half = 0; half < 2; ++half) {
+    const int blk = half == 0 ? nblk - 1 - pair : pair;
+    if (half == 1 && blk == nblk - 1 - pair) break;  // the middle block of an odd count, done once
+    const int r0 = blk * 128;
+    const int tmax_blk = min(T - 1, (min(r0 + 127, rows - 1)) / G);
+    const int64_t nkeys = P + tmax_blk + 1;
+    const int nsteps = (int)((nkeys + kRowsKeys - 1) / kRowsKeys);
+    const int iters = (nsteps + 1) / 2;
+    const int rt0 = r0 + 32 * tile;
+    const bool tile_live = rt0 < rows;
+    const int64_t tile_last_key = tile_live ? P + min(T - 1, min(rt0 + 31, rows - 1) / G) : -1;
+    const int64_t tile_first_vis = P + (int64_t)(min(rt0, rows - 1) / G);  // keys <= this: every row sees them
+    const int r = rt0 + ln;
+    const int rr = min(r, rows - 1);
+    const int t = rr / G;
+    const int64_t kvis = P + t;  // this lane's row sees keys <= kvis
+    u32x4_t qf[8];
+    {
+      const uint16_t* qrow = q + ((int64_t)t * nh + kvh * G + rr % G) * HD + 8 * g;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) qf[j] = *(const u32x4_t*)(qrow + 16 * j);
+    }
+    // the rounded scores of a step: s[sb][i] is key kb0 + 32 sb + 8 (i / 4) + 4 g + i % 4 of row r
+    auto scores = [&](const uint8_t* kbp, int64_t kb0, f32x16_t (&s)[2]) {
+#pragma unroll
+      for (int sb = 0; sb < 2; ++sb)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s[sb][i] = 0.f;
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+#pragma unroll
+        for (int sb = 0; sb < 2; ++sb) {
+          const u32x4_t kf = *(const u32x4_t*)(kbp + swz(32 * sb + ln, 2 * j + g));
+          if constexpr (DT == PE_DTYPE_F16)
+            s[sb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, kf),
+                                                           __builtin_bit_cast(f16x8_t, qf[j]), s[sb], 0, 0, 0);
+          else
+            s[sb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, kf),
+                                                            __builtin_bit_cast(bf16x8_t, qf[j]), s[sb], 0, 0, 0);
+        }
+      const bool whole = kb0 + kRowsKeys - 1 <= tile_first_vis;  // visible to every row of the tile
+      const uint64_t win = causal_window(kb0, kvis) >> (4 * g);
+#pragma unroll
+      for (int sb = 0; sb < 2; ++sb)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          s[sb][i] = eager_scaled<DT>(E::round(s[sb][i]));
+          if (!whole) s[sb][i] = ((win >> (32 * sb + 8 * (i >> 2) + (i & 3))) & 1ull) ? s[sb][i] : kEagerMasked;
+        }
+    };
+    // whether this wave's tile sees a key of its step of iteration `it` (wave-uniform)
+    auto sees = [&](int it) {
+      const int step = 2 * it + kg;
+      return tile_live && step < nsteps && (int64_t)step * kRowsKeys <= tile_last_key;
+    };
+    float m = kInitMax, l = 0.f;
+
+    __syncthreads();  // the previous block's buffers and hand-over are read by every wave
+    __builtin_amdgcn_s_waitcnt(0);  // Q has landed: no wait of the compiler's covers the ring's loads
+    // ---- pass 1: the row's max and sum
+    issue_k(0);
+    for (int it = 0; it < iters; ++it) {
+      __builtin_amdgcn_s_waitcnt(0);  // this wave's loads of iteration it have landed
+      __syncthreads();                // everyone's have, and iteration it - 1's buffers are free
+      if (it + 1 < iters) issue_k(it + 1);
+      if (!sees(it)) continue;
+      f32x16_t s[2];
+      scores(smem + (2 * (it & 1) + kg) * kRowsStepBytes, (int64_t)(2 * it + kg) * kRowsKeys, s);
+      float bmax = kEagerMasked;
+#pragma unroll
+      for (int sb = 0; sb < 2; ++sb)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) bmax = fmaxf(bmax, s[sb][i]);
+      bmax = fmaxf(bmax, __shfl_xor(bmax, 32, 64));
+      const float mnew = fmaxf(m, bmax);
+      float psum = 0.f;
+#pragma unroll
+      for (int sb = 0; sb < 2; ++sb)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) psum += exp_neg(s[sb][i] - mnew);
+      psum += __shfl_xor(psum, 32, 64);
+      l = l * exp_neg(m - mnew) + psum;
+      m = mnew;
+    }
+    if (g == 0) {
+      s_ml[((kg * 4 + tile) * 32 + ln) * 2] = m;
+      s_ml[((kg * 4 + tile) * 32 + ln) * 2 + 1] = l;
+    }
+    __syncthreads();  // pass 1's buffers are free too
+    issue_kv(0);
+    const float m0 = s_ml[(tile * 32 + ln) * 2], m1 = s_ml[((4 + tile) * 32 + ln) * 2];
+    const float M = fmaxf(m0, m1);
+    const float invL = 1.0f / (s_ml[(tile * 32 + ln) * 2 + 1] * exp_neg(m0 - M) +
+                               s_ml[((4 + tile) * 32 + ln) * 2 + 1] * exp_neg(m1 - M));
+    // ---- pass 2: O = sum_j round(exp(s_j - M) / L) v_j
+    f32x16_t o[4];
+#pragma unroll
+    for (int h = 0; h < 4; ++h)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) o[h][i] = 0.f;
+    for (int it = 0; it < iters; ++it) {
+      __builtin_amdgcn_s_waitcnt(0);
+      __syncthreads();
+      if (it + 1 < iters) issue_kv(it + 1);
+      if (!sees(it)) continue;
+      const uint8_t* kbp = smem + (2 * (it & 1) + kg) * kRowsStepBytes;
+      const uint8_t* vbp = kbp + 16384;
+      f32x16_t s[2];
+      scores(kbp, (int64_t)(2 * it + kg) * kRowsKeys, s);
+      uint32_t pb[2][8];
+#pragma unroll
+      for (int sb = 0; sb < 2; ++sb)
+#pragma unroll
+        for (int i = 0; i < 16; i += 2)
+          pb[sb][i >> 1] = pack2_16<DT>(exp_neg(s[sb][i] - M) * invL, exp_neg(s[sb][i + 1] - M) * invL);
+      const int qg = lane >> 4, jl = lane & 15;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const int sb = c >> 1, cq = c & 1;
+        u32x4_t bp;
+        bp[0] = pb[sb][4 * cq + 0];
+        bp[1] = pb[sb][4 * cq + 1];
+        bp[2] = pb[sb][4 * cq + 2];
+        bp[3] = pb[sb][4 * cq + 3];
+        const int kb = 16 * c + 4 * (qg >> 1) + (jl >> 2);
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+          const int db = 32 * h + 16 * (qg & 1) + 4 * (jl & 3);
+          typedef short s4v_t __attribute__((__vector_size__(4 * sizeof(short))));
+          typedef __attribute__((address_space(3))) s4v_t lds_s4v_t;
+          const s4v_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+              (lds_s4v_t*)(vbp + swz(kb, db >> 3) + (db & 7) * 2));
+          const s4v_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+              (lds_s4v_t*)(vbp + swz(kb + 8, db >> 3) + (db & 7) * 2));
+          const uint2 l2 = __builtin_bit_cast(uint2, lo), h2 = __builtin_bit_cast(uint2, hi);
+          u32x4_t a;
+          a[0] = l2.x;
+          a[1] = l2.y;
+          a[2] = h2.x;
+          a[3] = h2.y;
+          if constexpr (DT == PE_DTYPE_F16)
+            o[h] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a),
+                                                          __builtin_bit_cast(f16x8_t, bp), o[h], 0, 0, 0);
+          else
+            o[h] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a),
+                                                           __builtin_bit_cast(bf16x8_t, bp), o[h], 0, 0, 0);
+        }
+      }
+    }
+    __syncthreads();  // every wave is done with the step buffers
+    float* mo = (float*)smem + (tile * 64 + lane) * kRowsMergeStride;  // group 1 hands its sums to group 0
+    if (kg == 1) {
+#pragma unroll
+      for (int h = 0; h < 4; ++h)
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          *(f32x4_t*)&mo[16 * h + 4 * c] = f32x4_t{o[h][4 * c], o[h][4 * c + 1], o[h][4 * c + 2], o[h][4 * c + 3]};
+    }
+    __syncthreads();
+    if (kg == 0 && tile_live && r < rows) {
+      // o[h][4 c .. 4 c + 3] are dims 32 h + 8 c + 4 g + 0..3 of row r
+      const int col0 = (kvh * G + r % G) * HD;
+      typedef typename E::T Te;
+#pragma unroll
+      for (int h = 0; h < 4; ++h)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const f32x4_t o1 = *(const f32x4_t*)&mo[16 * h + 4 * c];
+          float o4[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o4[i] = o[h][4 * c + i] + o1[i];
+          const int col = col0 + 32 * h + 8 * c + 4 * g;
+          if (out_units)
+            Vec4<DT>::store((Te*)out + xtile_index(t, col, out_units), o4);
+          else if ((ld_out & 3) || ((uintptr_t)out & 7)) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) E::store((Te*)out, (int64_t)t * ld_out + col + i, o4[i]);
+          } else {
+            Vec4<DT>::store((Te*)out + (int64_t)t * ld_out + col, o4);
+          }
+        }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Batched tree attention with many rows per KV head (GQA batches)
 // ---------------------------------------------------------------------------
 // Sequence b's rows of a KV head are its T_b nodes x G query heads (row r =
@@ -1937,6 +2207,8 @@ extern "C" int64_t pe_attention_workspace_bytes(int T, int nh, int nkv, int hd, 
   return attention_workspace_bytes(T, nh, nkv, hd, kv_len, dtype, PE_ATTN_SDPA);
 }
 
+bool pe_internal_eager_tiles(int T, int mask_mode) { return mask_mode == PE_MASK_CAUSAL && T >= kRowsMinNodes; }
+
 int pe_internal_tree_attention(const void* q, const void* k_cache, const void* v_cache, int64_t cache_cap, int nh,
                                int nkv, int hd, int T, int64_t P, int mask_mode, const uint64_t* bits, int words,
                                float scale, int dtype, void* out, int64_t ld_out, int out_units, void* workspace,
@@ -1951,7 +2223,7 @@ int pe_internal_tree_attention(const void* q, const void* k_cache, const void* v
   const int64_t S = P + T;
   if (attn_mode != PE_ATTN_SDPA && attn_mode != PE_ATTN_EAGER) return PE_ERR_ARG;
   const int eager = attn_mode == PE_ATTN_EAGER;
-  if (eager && out_units) return PE_ERR_ARG;
+  if (eager && out_units && !pe_internal_eager_tiles(T, mask_mode)) return PE_ERR_ARG;
   if (workspace_bytes < attention_workspace_bytes(T, nh, nkv, hd, S, dtype, attn_mode)) return PE_ERR_WORKSPACE;
   if (dtype != PE_DTYPE_F32 && hd == 128 && !eager && mask_mode == PE_MASK_CAUSAL && T >= kRowsMinNodes) {
     // many causal rows (a prefill): row blocks in balanced pairs, no key splits
@@ -1996,8 +2268,21 @@ int pe_internal_tree_attention(const void* q, const void* k_cache, const void* v
     return PE_OK;
   }
   if (eager && dtype != PE_DTYPE_F32 && hd == 128) {
-    // the matrix-core eager kernel: every key of a row tile in one workgroup
+    // the matrix-core eager kernels: every key of a row tile in one workgroup
     if (cache_cap >= kAttnMaxCap) return PE_ERR_ARG;
+    if (pe_internal_eager_tiles(T, mask_mode)) {
+      const int nblk = (T * (nh / nkv) + 127) / 128, npair = (nblk + 1) / 2;
+      if (dtype == PE_DTYPE_BF16)
+        attn_eager_rows_kernel<PE_DTYPE_BF16><<<nkv * npair, 64 * kRowsWaves, 0, st>>>(
+            (const uint16_t*)q, (const uint16_t*)k_cache, (const uint16_t*)v_cache, cache_cap, nh, nkv, T, P, nblk,
+            npair, out, ld_out, out_units);
+      else
+        attn_eager_rows_kernel<PE_DTYPE_F16><<<nkv * npair, 64 * kRowsWaves, 0, st>>>(
+            (const uint16_t*)q, (const uint16_t*)k_cache, (const uint16_t*)v_cache, cache_cap, nh, nkv, T, P, nblk,
+            npair, out, ld_out, out_units);
+      PE_CHECK_LAUNCH();
+      return PE_OK;
+    }
     const dim3 grid(nkv, 1, (T * (nh / nkv) + 31) / 32);
     if (dtype == PE_DTYPE_BF16)
       attn_eager_kernel<PE_DTYPE_BF16><<<grid, 64 * kAttnWaves, 0, st>>>(

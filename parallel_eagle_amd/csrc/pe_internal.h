@@ -115,6 +115,8 @@ PE_INTERNAL int pe_internal_tree_attention(const void* q, const void* k_cache, c
                                            const uint64_t* bits, int words, float scale, int dtype, void* out,
                                            int64_t ld_out, int out_units, void* workspace, int64_t workspace_bytes,
                                            int* counters, hipStream_t st, int attn_mode = PE_ATTN_SDPA);
+// Whether an eager call of T nodes may write A-tiled output (16-bit, hd == 128).
+PE_INTERNAL bool pe_internal_eager_tiles(int T, int mask_mode);
 // Workspace of pe_internal_tree_attention in the given PE_ATTN_* mode.
 PE_INTERNAL int64_t attention_workspace_bytes(int T, int nh, int nkv, int hd, int64_t kv_len, int dtype,
                                               int attn_mode);

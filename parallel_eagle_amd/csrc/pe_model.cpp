@@ -299,7 +299,8 @@ int forward_prefill(const pe_model_desc* m, const pe_pass_args* a, const Prefill
                                      a->status, st));
     PE_TRY(copy_repeats(0, f0));
   }
-  const bool eager = m->attn_mode == PE_ATTN_EAGER;  // writes row-major output, packed afterwards
+  // eager attention of fewer rows writes row-major output, packed afterwards
+  const bool eager = m->attn_mode == PE_ATTN_EAGER && !pe_internal_eager_tiles(M, PE_MASK_CAUSAL);
   for (int l = 0; l < L; ++l) {
     void* kc = (char*)a->k_cache + l * layer_stride;
     void* vc = (char*)a->v_cache + l * layer_stride;
