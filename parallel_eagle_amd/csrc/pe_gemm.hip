@@ -1420,7 +1420,7 @@ __global__ __launch_bounds__(kWaves * 64, 3) void dense_gemm_kernel(const uint16
 
 // fp32 linear (VALU), K % 4 == 0 and 16-byte aligned rows: one wave per four
 // output columns (with SwiGLU their gate and up weight rows) and eight rows of
-// X, 16 lanes per column. A lane takes four consecutive k of every 64, so a
+// X (one for a single row), 16 lanes per column. A lane takes four consecutive k of every 64, so a
 // weight load is four 256-byte runs and an X load is shared by the columns;
 // each of its sums keeps the four k apart until the end (chains of K / 64
 // additions), and the 16 lanes' sums are added by a DPP butterfly, after which
@@ -1438,33 +1438,33 @@ __device__ __forceinline__ float row16_sum(float v) {
   return v;
 }
 
-template <bool SW>
+template <bool SW, int R>
 __global__ __launch_bounds__(64) void f32_gemm_vec_kernel(const float* __restrict__ X, int64_t ldx, int M, int K,
                                                           const float* __restrict__ W, int n_out, EpiArgs e) {
   const int lane = threadIdx.x, l16 = lane & 15;
   const int col = blockIdx.x * 4 + (lane >> 4);
-  const int m0 = blockIdx.y * 8;
-  const int nrow = min(8, M - m0);
+  const int m0 = blockIdx.y * R;
+  const int nrow = min(R, M - m0);
   const int wcol = min(col, n_out - 1);
   const int wrow = SW ? (wcol >> 5) * 64 + (wcol & 31) : wcol;
   const float* wg = W + (int64_t)wrow * K;
   const float* wu = wg + 32 * (int64_t)K;
-  f32x4_t a[8], b[8];
+  f32x4_t a[R], b[R];
 #pragma unroll
-  for (int r = 0; r < 8; ++r) a[r] = b[r] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int r = 0; r < R; ++r) a[r] = b[r] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   // kStep k-steps of 64 at a time, every load of them issued before the first
   // use (left to itself the compiler waits for each X row in turn); a lane past
   // K reads the row's first piece and skips it
-  constexpr int kStep = SW ? 2 : 4;
+  constexpr int kStep = R == 1 ? 8 : SW ? 2 : 4;
   for (int k0 = l16 * 4; k0 - l16 * 4 < K; k0 += 64 * kStep) {
-    f32x4_t w1[kStep], w2[kStep], x[kStep][8];
+    f32x4_t w1[kStep], w2[kStep], x[kStep][R];
 #pragma unroll
     for (int u = 0; u < kStep; ++u) {
       const int k = k0 + 64 * u < K ? k0 + 64 * u : 0;
       w1[u] = *(const f32x4_t*)(wg + k);
       if constexpr (SW) w2[u] = *(const f32x4_t*)(wu + k);
 #pragma unroll
-      for (int r = 0; r < 8; ++r)  // rows past M repeat the last
+      for (int r = 0; r < R; ++r)  // rows past M repeat the last
         x[u][r] = *(const f32x4_t*)(X + (int64_t)(m0 + min(r, nrow - 1)) * ldx + k);
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -1472,7 +1472,7 @@ __global__ __launch_bounds__(64) void f32_gemm_vec_kernel(const float* __restric
     for (int u = 0; u < kStep; ++u) {
       if (k0 + 64 * u >= K) break;
 #pragma unroll
-      for (int r = 0; r < 8; ++r)
+      for (int r = 0; r < R; ++r)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           a[r][i] = fmaf(x[u][r][i], w1[u][i], a[r][i]);
@@ -1482,7 +1482,7 @@ __global__ __launch_bounds__(64) void f32_gemm_vec_kernel(const float* __restric
   }
   float va = 0.f, vb = 0.f;
 #pragma unroll
-  for (int r = 0; r < 8; ++r) {
+  for (int r = 0; r < R; ++r) {
     const float sa = row16_sum((a[r][0] + a[r][1]) + (a[r][2] + a[r][3]));
     va = l16 == r ? sa : va;
     if constexpr (SW) {
@@ -2366,10 +2366,16 @@ extern "C" int pe_dense_gemm(const void* x, int64_t ldx, int M, int K, const voi
     const int n_out = epilogue == PE_EPI_SWIGLU ? N / 2 : N;
     dim3 grid((n_out + 3) / 4, (M + 7) / 8);
     const bool vec = K % 4 == 0 && ldx % 4 == 0 && (((uintptr_t)x | (uintptr_t)w) & 15) == 0;
-    if (vec && epilogue == PE_EPI_SWIGLU)
-      f32_gemm_vec_kernel<true><<<grid, 64, 0, st>>>((const float*)x, ldx, M, K, (const float*)w, n_out, e);
-    else if (vec)
-      f32_gemm_vec_kernel<false><<<grid, 64, 0, st>>>((const float*)x, ldx, M, K, (const float*)w, n_out, e);
+#define PE_F32_VEC(R)                                                                                            \
+  do {                                                                                                           \
+    if (epilogue == PE_EPI_SWIGLU)                                                                               \
+      f32_gemm_vec_kernel<true, R><<<grid, 64, 0, st>>>((const float*)x, ldx, M, K, (const float*)w, n_out, e);  \
+    else                                                                                                         \
+      f32_gemm_vec_kernel<false, R><<<grid, 64, 0, st>>>((const float*)x, ldx, M, K, (const float*)w, n_out, e); \
+  } while (0)
+    if (vec && M == 1) PE_F32_VEC(1);
+    else if (vec) PE_F32_VEC(8);
+#undef PE_F32_VEC
     else if (epilogue == PE_EPI_SWIGLU)
       f32_gemm_kernel<true><<<grid, 256, 0, st>>>((const float*)x, ldx, M, K, (const float*)w, n_out, e);
     else

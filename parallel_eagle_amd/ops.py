@@ -123,8 +123,14 @@ def gemm_workspace_bytes(m: int, n: int, k: int, nf4: bool, dtype: torch.dtype, 
                                              dcode(dtype), epilogue))
 
 
+COUNTER_BYTES = 32768  # the arrival counters at the head of a workspace, zero before its first use
+
+
 def _workspace(nbytes: int, device) -> torch.Tensor:
-    return torch.zeros(max(nbytes, 256), dtype=torch.uint8, device=device)
+    """A workspace for one call: only its counters need a value (the rest is written before it is read)."""
+    ws = torch.empty(max(nbytes, 256), dtype=torch.uint8, device=device)
+    ws[:COUNTER_BYTES].zero_()
+    return ws
 
 
 def linear(x: torch.Tensor, n: int, *, nf4: tuple | None = None, dense: torch.Tensor | None = None,
@@ -301,7 +307,7 @@ def tree_attention_batch(q, k_cache, v_cache, seq_row0, seq_prefix, bits, scale,
          "q and the caches must be contiguous with 128-dim heads")
     need = int(lib().pe_attention_batch_workspace_bytes(max_rows, nh, nkv, max_prefix + max_rows, b))
     if workspace is None:
-        workspace = torch.zeros(need, dtype=torch.uint8, device=q.device)
+        workspace = _workspace(need, q.device)
     out = torch.empty((m, nh * hd), dtype=q.dtype, device=q.device)
     check(lib().pe_tree_attention_batch(ptr(q), ptr(k_cache), ptr(v_cache), cap, nkv * cap * hd, nh, nkv, max_rows,
                                         max_prefix, b, ptr(seq_row0), ptr(seq_prefix), ptr(bits), bits.shape[1],
