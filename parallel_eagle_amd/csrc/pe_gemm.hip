@@ -837,20 +837,21 @@ __device__ __forceinline__ void bigws_consumer(uint8_t* smem, const uint16_t* __
     for (int mt = 0; mt < MA; ++mt)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[nt][mt][r] = 0.f;
-  // X fragments in a ring of four k-steps, two k-steps ahead of their MFMAs
-  u32x4_t x[4][MA];
+  // X fragments in a ring of eight k-steps, kLA k-steps ahead of their MFMAs
+  // without a break at a unit's end (the last unit asks for its own k-steps
+  // again). X comes from L2 and the consumers wait for it: the four products
+  // of a 7B layer at 150 / 208 rows took 127.0 / 137.5 us with two k-steps
+  // ahead that started anew with each unit, and take 124.8 / 133.3 with two,
+  // 120.0 / 131.1 with four and 118.4 / 131.7 with six (234 VGPRs of the 256).
+  constexpr int kLA = 6;
+  u32x4_t x[8][MA];
   auto load_x = [&](int p, int s) {
 #pragma unroll
     for (int mt = 0; mt < NMT; ++mt)
-      x[s & 3][mt] = *(const u32x4_t*)(X + ((((int64_t)(mt0 + mt) * NP + p) * 8 + s) * 64 + lane) * 8);
-  };
-  auto first_x = [&](int p) {
-    load_x(p, 0);
-    load_x(p, 1);
+      x[s & 7][mt] = *(const u32x4_t*)(X + ((((int64_t)(mt0 + mt) * NP + p) * 8 + s) * 64 + lane) * 8);
   };
   // relative unit t from ring slot t % 2: the four B fragments of k-step
-  // s + 1 are requested before the MFMAs of k-step s; the next unit's first
-  // X k-steps are requested before the round's barrier
+  // s + 1 are requested before the MFMAs of k-step s
   auto multiply = [&](int t) {
     const u32x4_t* src = bufs + (t & 1) * kBigNT * 8 * 64 + lane;
     u32x4_t b[2][kBigNT];
@@ -862,17 +863,17 @@ __device__ __forceinline__ void bigws_consumer(uint8_t* smem, const uint16_t* __
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
       if (NMT > 0 && s + 1 < 8) load_b(s + 1);
-      if (s + 2 < 8) load_x(u0 + t, s + 2);
+      load_x(min(u0 + t + ((s + kLA) >> 3), u1 - 1), (s + kLA) & 7);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int nt = 0; nt < kBigNT; ++nt)
 #pragma unroll
-        for (int mt = 0; mt < NMT; ++mt) acc[nt][mt] = mfma16<PE_DTYPE_BF16>(x[s & 3][mt], b[s & 1][nt], acc[nt][mt]);
+        for (int mt = 0; mt < NMT; ++mt) acc[nt][mt] = mfma16<PE_DTYPE_BF16>(x[s & 7][mt], b[s & 1][nt], acc[nt][mt]);
       __builtin_amdgcn_sched_barrier(0);
     }
-    if (t + 1 < n) first_x(u0 + t + 1);
   };
-  first_x(u0);
+#pragma unroll
+  for (int s = 0; s < kLA; ++s) load_x(u0, s);
   lds_barrier();
   for (int t = 0; t < n; t += 2) {
     multiply(t);
