@@ -2247,10 +2247,13 @@ int pe_internal_many_swiglu(int wfmt, int dtype, const void* x_tiled, int M, int
   return pe_internal_many_linear(wfmt, dtype, x_tiled, M, K, w, wabs, N, partial, partial_bytes, splits, st);
 }
 
-// A dense 16-bit pe_dense_gemm of more than 64 rows without bias or residual
-// packs X A-tiled into its workspace and runs the many-row kernel.
+// A dense 16-bit pe_dense_gemm of more than 256 rows without bias or residual
+// packs X A-tiled into its workspace and runs the many-row kernel. Up to 256
+// rows it stays on the 64-row launches, though the many-row kernel would be
+// faster (150 x 32000 x 4096: 63 us), because its logits then equal
+// pe_dense_gemm_argmax's bit for bit.
 static bool dense_many_rows(int M, int N, int K, int epilogue, const void* bias) {
-  return M > kMaxChunkRows && epilogue == PE_EPI_STORE && !bias && K % 128 == 0 && N % (32 * kBigNT) == 0;
+  return M > 256 && epilogue == PE_EPI_STORE && !bias && K % 128 == 0 && N % (32 * kBigNT) == 0;
 }
 
 extern "C" int64_t pe_gemm_workspace_bytes(int M, int N, int K, int wfmt, int dtype, int epilogue) {
