@@ -171,9 +171,9 @@ constexpr int kFusedChunk = 64;  // rows per fused pass (causal passes are chunk
 // append for q/k/v, residual + RMSNorm (with the captures) after o and down;
 // gate/up stores the SwiGLU activation itself where it runs unsplit.
 // Attention runs once over all rows, causally. (150 rows at the 7B width over
-// 900 cached ones, four layers of fp32-absmax weights: 1346 us as three
-// 64-row chunks of the fused pass, each of which streams and dequantises every
-// weight.)
+// 900 cached ones, four layers of fp32-absmax weights: 742 us, and 1317 us as
+// three 64-row chunks of the fused pass, each of which streams and dequantises
+// every weight.)
 // ---------------------------------------------------------------------------
 constexpr int kPrefillMinRows = kFusedChunk + 1;
 bool prefill_path(const pe_model_desc* m, int M, int mask_mode) {
@@ -203,7 +203,7 @@ struct PrefillLayout {
 PrefillLayout make_prefill_layout(const pe_model_desc* m, int M, int64_t kv_len) {
   PrefillLayout L;
   const int64_t H = m->hidden, qd = (int64_t)m->num_heads * m->head_dim;
-  const int64_t ip = m->intermediate_padded;
+  const int64_t nqkv = qd + 2ll * m->num_kv_heads * m->head_dim, ip = m->intermediate_padded;
   // offset 0: the pass's arrival counters, as in the fused layout (the GEMM
   // and attention counter slices rest at zero between passes, whichever path
   // ran last)
@@ -221,7 +221,12 @@ PrefillLayout make_prefill_layout(const pe_model_desc* m, int M, int64_t kv_len)
   L.attn = take(M * qd * 2);
   L.attn_t = take(xtile_bytes(M, (int)qd));
   L.act_t = take(xtile_bytes(M, (int)ip));
-  L.y_bytes = many_partials_bytes(m, M);
+  // Two splits of the widest linear hold the partials of every plan at model
+  // widths and grow with M, which the plans' own need does not (512 rows take
+  // more splits than 600): a workspace sized for a longer prompt serves every
+  // shorter one. Narrow models can need more.
+  const int64_t wide = std::max(std::max(nqkv, 2 * ip), H);
+  L.y_bytes = std::max(many_partials_bytes(m, M), M * wide * 8);
   L.y = take(L.y_bytes);
   L.attn_ws_bytes = align_up(attention_workspace_bytes(M, m->num_heads, m->num_kv_heads, m->head_dim, kv_len,
                                                        m->dtype, m->attn_mode));
@@ -485,14 +490,13 @@ int forward_fused(const pe_model_desc* m, const pe_pass_args* a, const Layout& L
 // ---------------------------------------------------------------------------
 // Batched verification: `batch` sequences, each a tree over its own cached
 // prefix, all M rows through every linear at once (each weight is streamed
-// once per 64-row chunk launch for the whole batch, not once per sequence);
-// attention runs over every sequence's own keys in one launch, and the q/k/v
-// epilogue appends each row's K/V at its own sequence's rows. Activations are
-// row-major (the A-tiled handoff is for single 64-row passes).
+// once for the whole batch, not once per sequence); attention runs over every
+// sequence's own keys in one launch, and the q/k/v epilogue (or the kernel that
+// sums its partials) appends each row's K/V at its own sequence's rows.
 // ---------------------------------------------------------------------------
 struct BatchLayout {
   int64_t gemm, gemm_bytes, h, xn, q, attn, act, kvoff, attn_ws, attn_ws_bytes;
-  bool big;                                   // the many-row NF4 path (A-tiled activations, split partials)
+  bool big;                                   // the many-row path (A-tiled activations, split partials)
   int64_t xn_t, attn_t, act_t, part, part_bytes;
   int64_t total;
 };
@@ -507,7 +511,8 @@ bool batch_big_path(const pe_model_desc* m, int M) {
          nqkv % 128 == 0;
 }
 
-BatchLayout make_batch_layout(const pe_model_desc* m, int M, int max_rows, int64_t max_kv_len, int batch) {
+BatchLayout make_batch_layout(const pe_model_desc* m, int M, int max_rows, int64_t max_kv_len, int batch,
+                              bool many = true) {
   BatchLayout L;
   const int es = esize(m->dtype);
   const int H = m->hidden, qd = m->num_heads * m->head_dim, ip = m->intermediate_padded;
@@ -536,7 +541,7 @@ BatchLayout make_batch_layout(const pe_model_desc* m, int M, int max_rows, int64
   L.attn_ws_bytes =
       align_up(pe_internal_attention_batch_bytes(max_rows, m->num_heads, m->num_kv_heads, max_kv_len, batch));
   L.attn_ws = take(L.attn_ws_bytes);
-  L.big = batch_big_path(m, M);
+  L.big = many && batch_big_path(m, M);
   L.xn_t = L.attn_t = L.act_t = L.part = L.part_bytes = 0;
   if (L.big) {
     L.xn_t = take(xtile_bytes(M, H));
@@ -547,6 +552,19 @@ BatchLayout make_batch_layout(const pe_model_desc* m, int M, int max_rows, int64
   }
   L.total = off;
   return L;
+}
+
+// The layout of a batched pass in `avail` bytes. A workspace that is too small
+// for the many-row path but holds the row-major one (one sized for another
+// number of rows: the partials of the many-row path do not grow with M alone)
+// runs the latter, except where the many-row path is the only one that
+// pe_forward_batch_workspace_bytes ever stood for (NF4 with fp16 absmax, up to
+// 256 rows).
+BatchLayout fit_batch_layout(const pe_model_desc* m, int M, int max_rows, int64_t max_kv_len, int batch,
+                             int64_t avail) {
+  const BatchLayout L = make_batch_layout(m, M, max_rows, max_kv_len, batch);
+  if (L.total <= avail || !L.big || (m->weight_format == PE_WFMT_NF4 && M <= 256)) return L;
+  return make_batch_layout(m, M, max_rows, max_kv_len, batch, false);
 }
 
 int64_t batch_layout_total(const pe_model_desc* m, int M, int max_rows, int64_t max_kv_len, int batch) {
@@ -745,14 +763,15 @@ extern "C" int pe_forward(const pe_model_desc* m, const pe_pass_args* a, void* s
       return forward_fused(m, a, Lo, st);
     }
     if (a->node_keys) return PE_ERR_ARG;
-    const BatchLayout Lb = make_batch_layout(m, M, a->max_seq_rows, a->prefix_len + a->max_seq_rows, a->batch);
+    const BatchLayout Lb =
+        fit_batch_layout(m, M, a->max_seq_rows, a->prefix_len + a->max_seq_rows, a->batch, a->workspace_bytes);
     if (a->workspace_bytes < Lb.total) return PE_ERR_WORKSPACE;
     return forward_batched(m, a, Lb, st);
   }
   const int64_t kv_len = a->prefix_len + M;
   if (a->mask_mode == PE_MASK_TREE && wide_tree_path(m, M)) {
     if (a->bits_words <= 0 || a->bits_words > PE_TREE_MAX_WORDS || M > 64 * a->bits_words) return PE_ERR_TREE;
-    const BatchLayout Lb = make_batch_layout(m, M, M, kv_len, 1);
+    const BatchLayout Lb = fit_batch_layout(m, M, M, kv_len, 1, a->workspace_bytes - kOneSeqBytes);
     if (a->workspace_bytes < Lb.total + kOneSeqBytes) return PE_ERR_WORKSPACE;
     int32_t* row0 = (int32_t*)((char*)a->workspace + Lb.total);
     int64_t* prefix = (int64_t*)((char*)row0 + 16);
@@ -768,8 +787,9 @@ extern "C" int pe_forward(const pe_model_desc* m, const pe_pass_args* a, void* s
   }
   if (prefill_path(m, M, a->mask_mode)) {
     const PrefillLayout Lp = make_prefill_layout(m, M, kv_len);
-    if (a->workspace_bytes < Lp.total) return PE_ERR_WORKSPACE;
-    return forward_prefill(m, a, Lp, st);
+    if (a->workspace_bytes >= Lp.total) return forward_prefill(m, a, Lp, st);
+    // up to four chunks' rows the chunked pass below runs in less
+    if (M > 4 * kFusedChunk) return PE_ERR_WORKSPACE;
   }
   const Layout Lo = make_layout(m, M, kv_len);
   if (m->qkv_layout == PE_QKV_ROPE_PAIRED) {

@@ -6,7 +6,7 @@ from dataclasses import replace
 import pytest
 import torch
 
-from parallel_eagle_amd import ops
+from parallel_eagle_amd import _lib, batch, ops
 from parallel_eagle_amd.batch import BatchKVCache, forward_tree_batch
 from parallel_eagle_amd.config import ModelShape
 from parallel_eagle_amd.model import DeviceModel
@@ -94,3 +94,40 @@ def test_batched_pass_equals_its_sequences_alone(target, trees):
         r0, r1 = info.row0[b], info.row0[b + 1]
         _close(logits[r0:r1], lg[0], target.dtype)
         _close(fused[r0:r1], fu[0], target.dtype)
+
+
+@pytest.mark.parametrize("rows", [65, 150, 256, 257])
+def test_causal_pass_in_the_workspace_of_a_chunk(target, rows, monkeypatch):
+    pos = torch.arange(rows, device=DEV)
+    ids = pos * 7 % SHAPE.vocab
+    want = target.forward_cached(ids, target.make_cache(), pos)[:2]
+    small = max(target.model.workspace_bytes(64, rows), target.model.workspace_bytes(rows % 64 or 64, rows))
+    monkeypatch.setattr(target, "_ws", torch.zeros(small, dtype=torch.uint8, device=DEV))
+    monkeypatch.setattr(type(target.model), "workspace_bytes", lambda self, m, kv_len: small)
+    if rows > 256:
+        with pytest.raises(_lib.PEError):
+            target.forward_cached(ids, target.make_cache(), pos)
+        return
+    got = target.forward_cached(ids, target.make_cache(), pos)[:2]
+    _close(got[0], want[0], target.dtype)
+    _close(got[1], want[1], target.dtype)
+
+
+@pytest.mark.parametrize("trees", [(40, 26), (60,) * 5])
+def test_batched_pass_in_a_smaller_workspace(target, trees, monkeypatch):
+    cache = BatchKVCache(target, len(trees), 256)
+    toks = [[(11 * i + b) % SHAPE.vocab for i in range(t)] for b, t in enumerate(trees)]
+    pars = [[-1] + [(i - 1) // 2 for i in range(1, t)] for t in trees]
+    for b in range(len(trees)):
+        p = torch.arange(20 + b, device=DEV)
+        target.forward_cached(p, cache.seq(b), p)
+    want = forward_tree_batch(target, toks, pars, cache)
+    need = batch.batch_workspace_bytes
+    monkeypatch.setattr(batch, "batch_workspace_bytes", lambda tm, t: need(tm, t) - 256)
+    if target.model.desc().weight_format == _lib.PE_WFMT_NF4 and sum(trees) <= 256:
+        with pytest.raises(_lib.PEError):
+            forward_tree_batch(target, toks, pars, cache)
+        return
+    got = forward_tree_batch(target, toks, pars, cache)
+    _close(got[0], want[0], target.dtype)
+    _close(got[1], want[1], target.dtype)

@@ -1,0 +1,22 @@
+"""pe_forward_workspace_bytes grows with the rows of a causal pass (65 rows and
+more), so a workspace of a long prompt serves every shorter one."""
+import ctypes as C
+
+import pytest
+
+from parallel_eagle_amd import _lib
+from test_abi import _desc_7b_nf4
+
+
+@pytest.mark.parametrize("fmt", [_lib.PE_WFMT_NF4, _lib.PE_WFMT_NF4_F32ABS, _lib.PE_WFMT_DENSE])
+def test_workspace_of_a_longer_prompt_serves_shorter_ones(fmt):
+    d = _desc_7b_nf4()
+    d.weight_format = fmt
+    lib = _lib.load()
+    # beyond the 256 nodes that a tree pass, which has its own layout, can have
+    rows = [257, 300, 400, 511, 512, 513, 600, 768, 769, 1024, 1025, 2000, 2048, 2049]
+    need = [lib.pe_forward_workspace_bytes(C.byref(d), m, 4096) for m in rows]
+    assert all(b >= a > 0 for a, b in zip(need, need[1:]))
+    # up to 256 rows a smaller workspace runs the chunked pass, so nothing that fits 257 rows is refused
+    chunk = lib.pe_forward_workspace_bytes(C.byref(d), 64, 4096)
+    assert chunk <= need[0]
