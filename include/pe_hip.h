@@ -467,7 +467,7 @@ int64_t pe_forward_batch_workspace_bytes(const pe_model_desc* m, int M, int max_
  * (src/pe/target.py:203-224 -> HF LlamaForCausalLM / Qwen2ForCausalLM forward,
  * modeling_llama.py:347-490): embeddings, L decoder layers with in-place KV
  * append, final norm, lm_head over all M rows, fused features.
- * A causal pass of more than 256 rows of a 16-bit model with 128-dim heads, NF4
+ * A causal pass of more than 64 rows of a 16-bit model with 128-dim heads, NF4
  * or dense (a prefill), runs every linear once over all rows in blocks of 256
  * rows on the matrix cores (each NF4 weight dequantised once per block inside
  * the GEMM) and attention once over all rows. Set PE_PREFILL_GEMM=0 to run such

@@ -8,7 +8,7 @@ over its own cached prefix of its own length:
 - ``BatchKVCache``: K, V [B][L][nkv][capacity][hd]; ``seq(b)`` is sequence b's
   cache with the TreeKVCache API (prefill it with ``forward_cached``);
 - ``forward_tree_batch``: one ``pe_forward`` over all B trees' rows (every
-  weight streamed once per 64-row chunk for the whole batch), each row's
+  weight streamed once for the whole batch), each row's
   K/V appended at its own sequence's rows, attention over each sequence's
   own keys in one launch;
 - ``accept_tree_batch``: the greedy walk of every sequence in one launch;

@@ -26,8 +26,10 @@
 // are in base 2 as well.
 //
 // The drafter's eager rounding (PE_ATTN_EAGER) at 16 bits: attn_eager_kernel,
-// the same tiles in two passes over the keys.
-// fp32 path: one block per (row, query head), scores in LDS, VALU arithmetic.
+// the same tiles in two passes over the keys, and attn_eager_rows_kernel for
+// the many rows of a context.
+// fp32 path: one block per (row, query head), scores in LDS, VALU arithmetic
+// (attn_f32_kernel; attn_generic_kernel for head sizes it does not take).
 
 #include "pe_common.h"
 #include "pe_internal.h"
