@@ -32,6 +32,7 @@
 // (attn_f32_kernel; attn_generic_kernel for head sizes it does not take).
 
 #include "pe_common.h"
+#include "pe_eager.h"
 #include "pe_internal.h"
 
 #include <type_traits>
@@ -877,33 +878,6 @@ __global__ __launch_bounds__(64 * kPairWaves, 1) void attn_pair_kernel(
     body(std::false_type());
 }
 
-// Arithmetic of the eager softmax. The masked score is finite (kEagerMasked):
-// exponentials of differences then need no special case.
-constexpr float kEagerMasked = -1.0e30f;
-
-// round(x / sqrt(128)) for x a value of the 16-bit type, the quotient in fp32
-// first (torch divides in fp32). The product with the reciprocal rounds to the
-// same bf16 for every bf16 value; fp16 needs the remainder's correction, which
-// gives the fp32 quotient itself (both checked for all 65536 values; only the
-// sign of a zero may differ).
-template <int DT>
-__device__ __forceinline__ float eager_scaled(float x) {
-  constexpr float kSqrt = 11.3137085f, kInv = 1.0f / kSqrt;
-  float q = x * kInv;
-  if constexpr (DT == PE_DTYPE_F16) q = fmaf(fmaf(-q, kSqrt, x), kInv, q);
-  return Elem<DT>::round(q);
-}
-
-// exp(x) for x <= 0 (finite): 2^(x log2 e), the product's rounding error put
-// back to first order, so that the result is as exact as v_exp_f32
-__device__ __forceinline__ float exp_neg(float x) {
-  constexpr float kHi = 1.44269502162933349609375f, kLo = 1.92596299112661746887e-8f, kLn2 = 0.693147180559945f;
-  const float t = x * kHi;
-  const float e = fmaf(x, kLo, fmaf(x, kHi, -t));
-  const float p = __builtin_amdgcn_exp2f(t);
-  return fmaf(p * kLn2, e, p);
-}
-
 // Eager attention on the matrix cores (PE_ATTN_EAGER, the drafter's attention,
 // src/pe/nn.py:84-87, 16-bit with hd = 128), one key split, so that a
 // workgroup sees every key of its rows: one workgroup = 8 waves = one (KV head,
@@ -911,7 +885,7 @@ __device__ __forceinline__ float exp_neg(float x) {
 // twice.
 //   Pass 1: S^T = K Q^T on MFMA; each score rounded as the reference rounds it
 //   (the product to the dtype, divided by sqrt(hd), to the dtype again; a
-//   masked key is very low); the row's max and the fp32 sum of exp(s - max) kept
+//   masked key is -inf); the row's max and the fp32 sum of exp(s - max) kept
 //   online; the waves' (max, sum) merged in LDS in wave order.
 //   Pass 2: the same scores again; each probability exp(s - M) / L rounded to
 //   the dtype, as softmax(...).to(q.dtype) leaves it, and multiplied by V on
@@ -1014,7 +988,7 @@ __global__ __launch_bounds__(64 * kAttnWaves, 1) void attn_eager_kernel(
     for (int i = 0; i < 16; ++i) {
       const int64_t kj = jb + 8 * (i >> 2) + 4 * g + (i & 3);
       const bool ok = kj < j1 && key_allowed(kj, P, t, mask_mode, nbits);
-      s[i] = ok ? eager_scaled<DT>(E::round(sc[i])) : kEagerMasked;
+      s[i] = ok ? E::round(eager_quotient<DT>(E::round(sc[i]))) : -INFINITY;
     }
   };
   constexpr std::integral_constant<int, 0> kK0{};
@@ -1027,7 +1001,7 @@ __global__ __launch_bounds__(64 * kAttnWaves, 1) void attn_eager_kernel(
     if constexpr (decltype(next_c)::value) load_k(jb + 32, 1 - KS);
     float s[16];
     scores(jb, KS, s);
-    float bmax = kEagerMasked;
+    float bmax = -INFINITY;
 #pragma unroll
     for (int i = 0; i < 16; ++i) bmax = fmaxf(bmax, s[i]);
     bmax = fmaxf(bmax, __shfl_xor(bmax, 32, 64));
@@ -1760,8 +1734,8 @@ __global__ __launch_bounds__(64 * kRowsWaves, 1) void attn_eager_rows_kernel(
       for (int sb = 0; sb < 2; ++sb)
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-          s[sb][i] = eager_scaled<DT>(E::round(s[sb][i]));
-          if (!whole) s[sb][i] = ((win >> (32 * sb + 8 * (i >> 2) + (i & 3))) & 1ull) ? s[sb][i] : kEagerMasked;
+          s[sb][i] = E::round(eager_quotient<DT>(E::round(s[sb][i])));
+          if (!whole) s[sb][i] = ((win >> (32 * sb + 8 * (i >> 2) + (i & 3))) & 1ull) ? s[sb][i] : -INFINITY;
         }
     };
     // whether this wave's tile sees a key of its step of iteration `it` (wave-uniform)
@@ -1782,7 +1756,7 @@ __global__ __launch_bounds__(64 * kRowsWaves, 1) void attn_eager_rows_kernel(
       if (!sees(it)) continue;
       f32x16_t s[2];
       scores(smem + (2 * (it & 1) + kg) * kRowsStepBytes, (int64_t)(2 * it + kg) * kRowsKeys, s);
-      float bmax = kEagerMasked;
+      float bmax = -INFINITY;
 #pragma unroll
       for (int sb = 0; sb < 2; ++sb)
 #pragma unroll
