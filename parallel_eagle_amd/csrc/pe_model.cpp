@@ -855,11 +855,12 @@ extern "C" int pe_forward(const pe_model_desc* m, const pe_pass_args* a, void* s
     return PE_OK;
   };
   // The norms gather the embeddings and store the captured hidden states
-  // (widths of whole 16-byte pieces at 16-byte aligned addresses; otherwise
-  // separate launches do).
+  // (widths of whole 16-byte pieces at 16-byte aligned addresses; otherwise,
+  // and in a model without layers, whose first norm is the final one, separate
+  // launches do).
   uintptr_t where = (uintptr_t)m->embed | (uintptr_t)m->final_norm | (uintptr_t)a->fused;
   for (int l = 0; l < m->num_layers; ++l) where |= (uintptr_t)m->attn_norm[l];
-  const bool fused_norms = pe_internal_norm_fits(H) && where % 16 == 0;
+  const bool fused_norms = m->num_layers > 0 && pe_internal_norm_fits(H) && where % 16 == 0;
   // x of `layer`'s hidden state h, normed by w into xn; captures h (layer's slots) and, final, xn (slot num_layers)
   auto norm = [&](int layer, const void* w, int mode, bool final) -> int {
     const int fh = final ? -1 : slot_of(layer), fx = final ? slot_of(layer) : -1;

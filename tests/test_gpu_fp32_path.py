@@ -93,3 +93,18 @@ def test_plain_pass_captures_every_hidden_state():
             assert torch.equal(parts[:, i], out.setdefault(ly, parts[:, i].clone()))
         assert torch.equal(logits[0], out.setdefault("logits", logits[0].clone()))
     assert not torch.equal(out[1], out[2])
+
+
+def test_pass_of_a_model_without_layers():
+    """Embeddings, the final norm and the lm_head alone."""
+    tm = TargetModel.synthetic(TINY_LLAMA, seed=2, device=DEV, keep_logical=True, norm_noise=0.1)
+    tm.model.desc().num_layers = 0
+    ids = torch.arange(3, 14, device=DEV)
+    logits = tm.forward_cached(ids, tm.make_cache(), torch.arange(11, device=DEV))[0][0]
+    h = tm.model.embed[ids].double()
+    x = h * torch.rsqrt(h.square().mean(-1, keepdim=True) + TINY_LLAMA.rms_eps) * tm.model.final_norm.double()
+    w = tm.model.lm_head_logical.double()
+    k = TINY_LLAMA.hidden
+    # the product's K roundings, and the norm's row sum (K / 256 + 12 of them) and two products
+    bound = (k + k / 256 + 20) * 2.0 ** -24 * (x.abs() @ w.abs().T)
+    assert bool(((logits.double() - x @ w.T).abs() <= bound).all())
