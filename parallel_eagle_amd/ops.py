@@ -24,7 +24,8 @@ def lib():
 
 
 def stream_ptr() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    """The current stream's handle (0.3 us; building a torch.cuda.Stream object for it takes 2.9 us of every call)."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def ptr(t: torch.Tensor | None) -> int | None:
@@ -124,11 +125,18 @@ def gemm_workspace_bytes(m: int, n: int, k: int, nf4: bool, dtype: torch.dtype, 
 
 
 COUNTER_BYTES = 32768  # the arrival counters at the head of a workspace, zero before its first use
+# Up to this size one torch.zeros is the cheaper call: 4.9 us of host time at any size up to 16 MiB, where an allocation
+# and a fill of the counters alone take 6.1 us. Calls with larger workspaces are mostly bound by the GPU's own time, in
+# which filling the counters alone is shorter: attention of one node over 16000 keys (2.2 MB) takes 24.1 us and 24.9
+# with all of it cleared, of 26 nodes over 4096 keys (4 MB) 19.9 and 21.4.
+ZEROED_BYTES = 2 << 20
 
 
 def _workspace(nbytes: int, device) -> torch.Tensor:
     """A workspace for one call: only its counters need a value (the rest is written before it is read)."""
-    ws = torch.empty(max(nbytes, 256), dtype=torch.uint8, device=device)
+    if nbytes <= ZEROED_BYTES:
+        return torch.zeros(max(nbytes, 256), dtype=torch.uint8, device=device)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
     ws[:COUNTER_BYTES].zero_()
     return ws
 

@@ -1,10 +1,12 @@
 """pe_forward_workspace_bytes grows with the rows of a causal pass (65 rows and
-more), so a workspace of a long prompt serves every shorter one."""
+more), so a workspace of a long prompt serves every shorter one. A call's own
+workspace: one dispatched operation while it is small, its counters zero."""
 import ctypes as C
 
 import pytest
+from torch.utils._python_dispatch import TorchDispatchMode
 
-from parallel_eagle_amd import _lib
+from parallel_eagle_amd import _lib, ops
 from test_abi import _desc_7b_nf4
 
 
@@ -20,3 +22,19 @@ def test_workspace_of_a_longer_prompt_serves_shorter_ones(fmt):
     # up to 256 rows a smaller workspace runs the chunked pass, so nothing that fits 257 rows is refused
     chunk = lib.pe_forward_workspace_bytes(C.byref(d), 64, 4096)
     assert chunk <= need[0]
+
+
+@pytest.mark.parametrize("nbytes", [0, 4096, ops.ZEROED_BYTES, ops.ZEROED_BYTES + 1])
+def test_workspace_of_one_call(nbytes):
+    calls = []
+
+    class Count(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            calls.append(func)
+            return func(*args, **(kwargs or {}))
+
+    with Count():
+        ws = ops._workspace(nbytes, "cpu")
+    assert ws.numel() == max(nbytes, 256) and int(ws[: ops.COUNTER_BYTES].count_nonzero()) == 0
+    if nbytes <= ops.ZEROED_BYTES:
+        assert len(calls) == 1
