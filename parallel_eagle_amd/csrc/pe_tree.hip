@@ -483,7 +483,7 @@ __global__ void kv_gather_kernel(uint8_t* __restrict__ kc, uint8_t* __restrict__
 }
 
 // Beam tree proposal (propose_tree, src/pe/decode/tree.py:34-55) in three
-// launches.
+// launches (two for short rows, see kShortRow).
 //   * draft_topk_kernel: one block per depth row. Every thread finds the best
 //     element of its share of the row; one wave then takes the row's top c_d
 //     tokens in (value descending, index ascending) order: the best of the
@@ -509,6 +509,11 @@ constexpr int kBeamThreads = 256;
 constexpr int kSlices = kArgThreads / 64;  // slices of 64 partial sums
 constexpr int kExpTile = 128;              // elements of a partial sum staged at a time
 constexpr int kExpThreads = 512;
+// Up to this row length draft_topk_kernel takes the sums itself, one thread per
+// partial sum, and the second launch is left out: five rows at two tokens each
+// take 15.5 us of 2048 elements with one launch less and 17.0 with it, 17.9 and
+// 18.0 of 16384, 20.8 and 19.0 of 32000.
+constexpr int64_t kShortRow = 16384;
 static_assert(kSlices <= PE_PROPOSE_MAX_WIDTH, "a row's slice sums are staged in its log-probability scratch");
 
 struct BeamShape {
@@ -542,7 +547,8 @@ __device__ __forceinline__ void wave_best(uint32_t& bk, int& bi) {
 template <int DT>
 __global__ __launch_bounds__(kArgThreads) void draft_topk_kernel(const typename Elem<DT>::T* __restrict__ logits,
                                                                  int64_t ld, int64_t V, BeamShape bs,
-                                                                 int32_t* __restrict__ tok_out, int32_t* status) {
+                                                                 int32_t* __restrict__ tok_out,
+                                                                 float* __restrict__ sums, int32_t* status) {
   const int d = blockIdx.x;
   const typename Elem<DT>::T* x = logits + (int64_t)d * ld;
   constexpr int kPer = 16 / sizeof(typename Elem<DT>::T);
@@ -556,8 +562,7 @@ __global__ __launch_bounds__(kArgThreads) void draft_topk_kernel(const typename 
   s_key[threadIdx.x] = bk;
   s_idx[threadIdx.x] = bi;
   nan = __syncthreads_or(nan);
-  if (threadIdx.x >= 64) return;
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x & 63;
   int32_t* out = tok_out + d * PE_PROPOSE_MAX_WIDTH;
   // the best of this lane's 16 shares (lane, lane + 64, ...)
   uint32_t lk = 0;
@@ -575,13 +580,34 @@ __global__ __launch_bounds__(kArgThreads) void draft_topk_kernel(const typename 
       }
     }
   };
-  scan();
+  uint32_t pk = 0;
+  int pi = -1;
+  if (threadIdx.x < 64) {
+    scan();
+    pk = lk;
+    pi = li;
+    wave_best(pk, pi);
+  }
+  if (sums) {
+    // a short row: partial sum t by thread t, slice w by wave w
+    __shared__ int s_first;
+    if (threadIdx.x == 0) s_first = pi;
+    __syncthreads();
+    const float mx = Elem<DT>::load(x, s_first);
+    float s = 0.f;
+    for (int64_t i = threadIdx.x; i < V; i += kArgThreads) s += expf(Elem<DT>::load(x, i) - mx);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    if (lane == 0) sums[d * PE_PROPOSE_MAX_WIDTH + (threadIdx.x >> 6)] = s;
+  }
+  if (threadIdx.x >= 64) return;
   const int c = bs.cand[d];
   for (int j = 0; j < c; ++j) {
-    uint32_t pk = lk;
-    int pi = li;
-    wave_best(pk, pi);
-    if (j == 0) {
+    if (j > 0) {
+      pk = lk;
+      pi = li;
+      wave_best(pk, pi);
+    } else {
       const float mx = Elem<DT>::load(x, pi);
       if (nan || !(mx > -INFINITY) || mx == INFINITY) {
         if (lane == 0) {
@@ -950,10 +976,13 @@ extern "C" int pe_propose_tree(const void* logits, int64_t ld, int k, int64_t V,
 #define PE_PROPOSE(D)                                                                                            \
   do {                                                                                                          \
     const Elem<D>::T* x = (const Elem<D>::T*)logits;                                                            \
-    draft_topk_kernel<D><<<k, kArgThreads, 0, st>>>(x, ld, V, bs, tok, status);                                  \
+    const bool short_row = V <= kShortRow;                                                                      \
+    draft_topk_kernel<D><<<k, kArgThreads, 0, st>>>(x, ld, V, bs, tok, short_row ? lp : nullptr, status);        \
     PE_CHECK_LAUNCH();                                                                                          \
-    draft_expsum_kernel<D><<<dim3(kSlices, k), kExpThreads, 0, st>>>(x, ld, V, tok, lp);                         \
-    PE_CHECK_LAUNCH();                                                                                          \
+    if (!short_row) {                                                                                           \
+      draft_expsum_kernel<D><<<dim3(kSlices, k), kExpThreads, 0, st>>>(x, ld, V, tok, lp);                       \
+      PE_CHECK_LAUNCH();                                                                                        \
+    }                                                                                                           \
     beam_kernel<D><<<1, kBeamThreads, 0, st>>>(x, ld, bs, lp, tok, node_tokens, parents, status);                \
     PE_CHECK_LAUNCH();                                                                                          \
   } while (0)

@@ -1,8 +1,8 @@
 """Parallel tree drafting with the API of src/pe/decode/tree.py:19-57.
 
 The drafter's logits stay on the device: the per-depth log_softmax, each depth's
-top candidates and the beam over depths run in two kernels (``pe_propose_tree``)
-instead of one ``.tolist()`` per depth and a Python sort. ``propose_tree`` keeps
+top candidates and the beam over depths run in two or three kernels
+(``pe_propose_tree``) instead of one ``.tolist()`` per depth and a Python sort. ``propose_tree`` keeps
 the reference's signature and list results; ``propose_tree_device`` returns the
 device tensors the verification pass takes, without waiting for the GPU.
 

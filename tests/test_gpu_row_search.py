@@ -68,3 +68,23 @@ def test_top_tokens_of_rows_with_many_ties(dtype, v, c, pad):
         ref = torch.log_softmax(x.double(), -1)[torch.from_numpy(want)]
         # a sum of v fp32 terms in 1024 partial sums: v / 1024 + 26 roundings of 2^-24, and a few of the logarithm
         assert bool(((lp[d].double() - ref).abs() <= (v / 1024 + 32) * 2.0 ** -24 * (1 + ref.abs())).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("v", [1, 63, 1024, 1025, 16384])
+def test_log_probabilities_do_not_depend_on_the_row_length_rule(dtype, v):
+    """A short row's sum is taken by the search's own launch: the same bits as for the same row followed by -inf up
+    to a length whose sums have a launch of their own (their exponentials are zeros)."""
+    gen = torch.Generator().manual_seed(v)
+    x = (torch.randn(2, v, generator=gen) * 3).to(dtype)
+    wide = torch.full((2, 20000), float("-inf"), dtype=dtype)
+    wide[:, :v] = x
+    c = min(v, 8)
+    out = []
+    for rows in (x, wide):
+        scratch = torch.zeros(2 * _lib.PE_PROPOSE_SCRATCH_PER_DEPTH, dtype=torch.uint8, device=DEV)
+        tokens, parents, status = ops.propose_tree(rows.to(DEV), [c] * 2, c, scratch=scratch)
+        assert int(status.item()) == 0
+        W = _lib.PE_PROPOSE_MAX_WIDTH
+        out.append((tokens.cpu(), parents.cpu(), scratch[: 2 * W * 4].view(torch.int32).view(2, W)[:, :c].cpu()))
+    assert all(torch.equal(a, b) for a, b in zip(*out))
