@@ -2179,6 +2179,14 @@ int64_t attention_workspace_bytes(int T, int nh, int nkv, int hd, int64_t kv_len
   return (int64_t)T * nh * kv_len * 4;
 }
 
+int64_t attention_reserve_bytes(int T, int nh, int nkv, int hd, int64_t kv_len, int dtype, int attn_mode) {
+  const int64_t b = attention_workspace_bytes(T, nh, nkv, hd, kv_len, dtype, attn_mode);
+  if (b <= 0 || dtype == PE_DTYPE_F32 || hd != 128 || attn_mode == PE_ATTN_EAGER) return b;
+  // calls with key splits: at most 256 workgroups of 32 rows in all
+  constexpr int64_t kSplitBytes = kAttnCounterBytes + 256 * 32 * (128 + 4) * 4;
+  return b > kSplitBytes ? b : kSplitBytes;
+}
+
 extern "C" int64_t pe_attention_workspace_bytes(int T, int nh, int nkv, int hd, int64_t kv_len, int dtype) {
   return attention_workspace_bytes(T, nh, nkv, hd, kv_len, dtype, PE_ATTN_SDPA);
 }

@@ -42,6 +42,7 @@
 #include "pe_common.h"
 #include "pe_internal.h"
 
+#include <algorithm>
 #include <cmath>
 #include <cstdlib>
 #include <type_traits>
@@ -2032,7 +2033,7 @@ namespace {
 struct BigPlan {
   int groups, units, S, pps;
 };
-BigPlan big_plan(int M, int N, int K) {
+BigPlan big_plan(int M, int N, int K, int max_splits = kMaxSplits) {
   BigPlan p;
   p.groups = N / (32 * kBigNT);
   p.units = K / 128;
@@ -2047,6 +2048,7 @@ BigPlan big_plan(int M, int N, int K) {
   if (S < 1) S = 1;
   if (forced > 0) S = forced;
   if (S > kMaxSplits) S = kMaxSplits;
+  if (S > max_splits) S = max_splits;
   if (S > p.units) S = p.units;
   if (S < 1) S = 1;
   p.pps = (p.units + S - 1) / S;
@@ -2208,27 +2210,45 @@ constexpr int kDenseMaxSplits = 8;
 
 bool pe_internal_many_fits(int N, int K) { return N > 0 && K >= 128 && N % (32 * kBigNT) == 0 && K % 128 == 0; }
 
-int64_t pe_internal_many_partials_bytes(int wfmt, int M, int N, int K) {
-  if (M <= 0 || !pe_internal_many_fits(N, K)) return 0;
-  const int S = pe_wfmt_nf4(wfmt) ? big_plan(M, N, K).S : dense_bigm_splits(M, N, K, kDenseMaxSplits);
+int64_t pe_internal_many_partials_bytes(int wfmt, int M, int N, int K, int max_splits) {
+  if (M <= 0 || max_splits < 1 || !pe_internal_many_fits(N, K)) return 0;
+  const int S = pe_wfmt_nf4(wfmt) ? big_plan(M, N, K, max_splits).S
+                                  : dense_bigm_splits(M, N, K, std::min(kDenseMaxSplits, max_splits));
   return (int64_t)S * M * N * 4;
 }
 
+int64_t pe_internal_many_reserve_bytes(int wfmt, int M, int N, int K) {
+  if (M <= 0 || !pe_internal_many_fits(N, K)) return 0;
+  if (!pe_wfmt_nf4(wfmt)) {
+    const int S = N % 256 ? 2 : std::max(1, std::min(kDenseMaxSplits, cu_count() / (N / 256)));
+    return (int64_t)std::min(M, 256) * N * S * 4;
+  }
+  // the plan changes with the blocks of 256 rows only
+  int64_t r = 0;
+  for (int rows = std::min(M, 256);; rows = std::min(M, rows + 256)) {
+    r = std::max(r, pe_internal_many_partials_bytes(wfmt, rows, N, K));
+    if (rows == M) return r;
+  }
+}
+
 int pe_internal_many_linear(int wfmt, int dtype, const void* x_tiled, int M, int K, const void* w, const void* wabs,
-                            int N, float* partial, int64_t partial_bytes, int* splits, hipStream_t st) {
-  if (!x_tiled || !w || !partial || !splits || M <= 0 || !pe_internal_many_fits(N, K)) return PE_ERR_ARG;
-  if (partial_bytes < pe_internal_many_partials_bytes(wfmt, M, N, K)) return PE_ERR_WORKSPACE;
+                            int N, float* partial, int64_t partial_bytes, int* splits, hipStream_t st,
+                            int max_splits) {
+  if (!x_tiled || !w || !partial || !splits || M <= 0 || max_splits < 1 || !pe_internal_many_fits(N, K))
+    return PE_ERR_ARG;
+  if (partial_bytes < pe_internal_many_partials_bytes(wfmt, M, N, K, max_splits)) return PE_ERR_WORKSPACE;
   if (!pe_wfmt_nf4(wfmt))
-    return pe_internal_dense_bigm(x_tiled, M, K, w, dtype, N, partial, N, st, true, splits, kDenseMaxSplits);
+    return pe_internal_dense_bigm(x_tiled, M, K, w, dtype, N, partial, N, st, true, splits,
+                                  std::min(kDenseMaxSplits, max_splits));
   if (!wabs) return PE_ERR_ARG;
-  const BigPlan p = big_plan(M, N, K);
+  const BigPlan p = big_plan(M, N, K, max_splits);
   *splits = p.S;
   return launch_bigws(wfmt, p, x_tiled, M, w, wabs, make_epi(kEpiPartial, M, N, nullptr, nullptr, 0, partial, N), st);
 }
 
 int pe_internal_many_swiglu(int wfmt, int dtype, const void* x_tiled, int M, int K, const void* w, const void* wabs,
                             int N, void* out, int out_units, float* partial, int64_t partial_bytes, int* splits,
-                            hipStream_t st) {
+                            hipStream_t st, int max_splits) {
   if (!x_tiled || !w || !out || !splits || M <= 0 || !pe_internal_many_fits(N, K) || out_units * 256 != N)
     return PE_ERR_ARG;
   *splits = 0;
@@ -2237,14 +2257,15 @@ int pe_internal_many_swiglu(int wfmt, int dtype, const void* x_tiled, int M, int
       return t256_launch(x_tiled, M, K, w, dtype, N, out, 0, kEpiTSwiglu, out_units, t256_plan(M, N, K, 1, false), st);
   } else {
     if (!wabs) return PE_ERR_ARG;
-    const BigPlan p = big_plan(M, N, K);
+    const BigPlan p = big_plan(M, N, K, max_splits);
     if (p.S == 1 && dtype == PE_DTYPE_BF16) {
       EpiArgs e = make_epi(PE_EPI_SWIGLU, M, N, nullptr, nullptr, 0, out, 0);
       e.out_units = out_units;
       return launch_bigws(wfmt, p, x_tiled, M, w, wabs, e, st);
     }
   }
-  return pe_internal_many_linear(wfmt, dtype, x_tiled, M, K, w, wabs, N, partial, partial_bytes, splits, st);
+  return pe_internal_many_linear(wfmt, dtype, x_tiled, M, K, w, wabs, N, partial, partial_bytes, splits, st,
+                                 max_splits);
 }
 
 // A dense 16-bit pe_dense_gemm of more than 256 rows without bias or residual

@@ -64,19 +64,25 @@ PE_INTERNAL int pe_internal_dense_bigm(const void* x_tiled, int M, int K, const 
                                        int* splits = nullptr, int max_splits = 1);
 // A pass's linear over many rows (more than 64, A-tiled X; pe_internal_many_fits
 // shapes) in any 16-bit weight format (PE_WFMT_*): fp32 split partials
-// [S][M][N], *splits receives S. NF4 weights are dequantised once per block of
-// 256 rows.
+// [S][M][N], *splits receives S, at most max_splits. NF4 weights are dequantised
+// once per block of 256 rows.
+// pe_internal_many_reserve_bytes grows with M, which the plans' own need does
+// not (512 rows can take more splits than 600): it holds every NF4 plan of up
+// to M rows and a round of workgroups of every dense one.
+constexpr int kManySplits = 1 << 30;  // no limit but the plan's own
 PE_INTERNAL bool pe_internal_many_fits(int N, int K);
-PE_INTERNAL int64_t pe_internal_many_partials_bytes(int wfmt, int M, int N, int K);
+PE_INTERNAL int64_t pe_internal_many_partials_bytes(int wfmt, int M, int N, int K, int max_splits = kManySplits);
+PE_INTERNAL int64_t pe_internal_many_reserve_bytes(int wfmt, int M, int N, int K);
 PE_INTERNAL int pe_internal_many_linear(int wfmt, int dtype, const void* x_tiled, int M, int K, const void* w,
                                         const void* wabs, int N, float* partial, int64_t partial_bytes, int* splits,
-                                        hipStream_t st);
+                                        hipStream_t st, int max_splits = kManySplits);
 // The same with the SwiGLU of an interleaved gate/up weight (N = 256 *
 // out_units): the GEMM stores the A-tiled activation itself and *splits = 0,
 // or it writes split partials (*splits = S) for pe_internal_swiglu_partials.
 PE_INTERNAL int pe_internal_many_swiglu(int wfmt, int dtype, const void* x_tiled, int M, int K, const void* w,
                                         const void* wabs, int N, void* out, int out_units, float* partial,
-                                        int64_t partial_bytes, int* splits, hipStream_t st);
+                                        int64_t partial_bytes, int* splits, hipStream_t st,
+                                        int max_splits = kManySplits);
 // Row-major 16-bit [M][K] (leading dimension ld) -> the A-tiled layout
 // (K % 128 == 0; rows past M of the last 32-row tile are written as zeros).
 PE_INTERNAL int pe_internal_to_xtile(const void* x, int64_t ld, int M, int K, void* out, hipStream_t st);
@@ -120,6 +126,8 @@ PE_INTERNAL bool pe_internal_eager_tiles(int T, int mask_mode);
 // Workspace of pe_internal_tree_attention in the given PE_ATTN_* mode.
 PE_INTERNAL int64_t attention_workspace_bytes(int T, int nh, int nkv, int hd, int64_t kv_len, int dtype,
                                               int attn_mode);
+// The same for every call of up to T nodes over up to kv_len keys (it grows with T).
+PE_INTERNAL int64_t attention_reserve_bytes(int T, int nh, int nkv, int hd, int64_t kv_len, int dtype, int attn_mode);
 
 // pe_attn.hip: tree attention of `batch` sequences in one launch (16-bit,
 // hd == 128): sequence b's query rows are [seq_row0[b], seq_row0[b+1]) of q,

@@ -221,15 +221,17 @@ PrefillLayout make_prefill_layout(const pe_model_desc* m, int M, int64_t kv_len)
   L.attn = take(M * qd * 2);
   L.attn_t = take(xtile_bytes(M, (int)qd));
   L.act_t = take(xtile_bytes(M, (int)ip));
-  // Two splits of the widest linear hold the partials of every plan at model
-  // widths and grow with M, which the plans' own need does not (512 rows take
-  // more splits than 600): a workspace sized for a longer prompt serves every
-  // shorter one. Narrow models can need more.
+  // fp32 split partials: a size that grows with M at every width, so that a
+  // workspace of a longer prompt serves every shorter one; a pass takes no more
+  // splits than fit (at least two of the widest linear)
   const int64_t wide = std::max(std::max(nqkv, 2 * ip), H);
-  L.y_bytes = std::max(many_partials_bytes(m, M), M * wide * 8);
+  const int wf = m->weight_format;
+  L.y_bytes = M * wide * 8;
+  for (const auto& s : {std::pair<int64_t, int64_t>(nqkv, H), {H, qd}, {2 * ip, H}, {H, ip}})
+    L.y_bytes = std::max(L.y_bytes, pe_internal_many_reserve_bytes(wf, M, (int)s.first, (int)s.second));
   L.y = take(L.y_bytes);
-  L.attn_ws_bytes = align_up(attention_workspace_bytes(M, m->num_heads, m->num_kv_heads, m->head_dim, kv_len,
-                                                       m->dtype, m->attn_mode));
+  L.attn_ws_bytes = align_up(
+      attention_reserve_bytes(M, m->num_heads, m->num_kv_heads, m->head_dim, kv_len, m->dtype, m->attn_mode));
   L.attn_ws = take(L.attn_ws_bytes);
   L.total = off;
   return L;
@@ -293,8 +295,9 @@ int forward_prefill(const pe_model_desc* m, const pe_pass_args* a, const Prefill
   // y[ys][M][N] (fp32 split partials) = x (A-tiled) . W^T over all rows
   const int wf = m->weight_format;
   int ys = 0;
+  auto fitting = [&](int N) { return (int)(Lp.y_bytes / ((int64_t)M * N * 4)); };  // splits
   auto linear = [&](const void* xt, int K, const void* w, const void* ab, int N) -> int {
-    return pe_internal_many_linear(wf, m->dtype, xt, M, K, w, ab, N, y, Lp.y_bytes, &ys, st);
+    return pe_internal_many_linear(wf, m->dtype, xt, M, K, w, ab, N, y, Lp.y_bytes, &ys, st, fitting(N));
   };
 
   {
@@ -322,7 +325,7 @@ int forward_prefill(const pe_model_desc* m, const pe_pass_args* a, const Prefill
     PE_TRY(pe_internal_residual_rmsnorm(y, ys, M, h, H, m->mlp_norm[l], m->rms_eps, m->norm_mode, m->dtype, nullptr, xn_t,
                                         nullptr, 0, nullptr, 0, st));
     PE_TRY(pe_internal_many_swiglu(wf, m->dtype, xn_t, M, H, m->w_gu[l], m->a_gu ? m->a_gu[l] : nullptr, 2 * ip, act_t,
-                                   ip / 128, y, Lp.y_bytes, &ys, st));
+                                   ip / 128, y, Lp.y_bytes, &ys, st, fitting(2 * ip)));
     if (ys > 0) PE_TRY(pe_internal_swiglu_partials(y, ys, M, 2 * ip, act_t, ip, ip / 128, m->dtype, st));
     PE_TRY(linear(act_t, ip, m->w_down[l], m->a_down ? m->a_down[l] : nullptr, H));
     const bool last = l + 1 == L;

@@ -19,8 +19,8 @@ SHAPE = ModelShape(name="small", num_layers=2, hidden=512, num_heads=4, num_kv_h
                    feature_layers=(0, 1, 2), max_positions=1024)
 
 
-def _target(fmt):
-    shape = SHAPE if fmt.startswith("nf4") else replace(SHAPE, weight_format="dense", dtype=fmt)
+def _target(fmt, shape=SHAPE):
+    shape = shape if fmt.startswith("nf4") else replace(shape, weight_format="dense", dtype=fmt)
     gen = torch.Generator(device=DEV).manual_seed(5)
     rnd = lambda *size, std=0.04: torch.randn(size, generator=gen, device=DEV) * std
     w = {"embed": rnd(shape.vocab, shape.hidden, std=1.0), "lm_head": rnd(shape.vocab, shape.hidden),
@@ -111,6 +111,20 @@ def test_causal_pass_in_the_workspace_of_a_chunk(target, rows, monkeypatch):
     got = target.forward_cached(ids, target.make_cache(), pos)[:2]
     _close(got[0], want[0], target.dtype)
     _close(got[1], want[1], target.dtype)
+
+
+@pytest.mark.parametrize("fmt", ["nf4-f16abs", "nf4-f32abs", "bfloat16"])
+def test_causal_pass_in_the_workspace_of_a_longer_one(fmt, monkeypatch):
+    """512 rows take more K splits than 513 at this width."""
+    tm = _target(fmt, replace(SHAPE, num_heads=8, num_kv_heads=8, intermediate=1408))
+    pos = torch.arange(512, device=DEV)
+    ids = pos * 7 % SHAPE.vocab
+    want = tm.forward_cached(ids, tm.make_cache(), pos)[:2]
+    longer = min(tm.model.workspace_bytes(m, 640) for m in range(513, 640))
+    monkeypatch.setattr(tm, "_ws", torch.zeros(longer, dtype=torch.uint8, device=DEV))
+    monkeypatch.setattr(type(tm.model), "workspace_bytes", lambda self, m, kv_len: longer)
+    got = tm.forward_cached(ids, tm.make_cache(), pos)[:2]
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
 
 
 @pytest.mark.parametrize("trees", [(40, 26), (60,) * 5])

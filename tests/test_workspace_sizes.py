@@ -24,6 +24,18 @@ def test_workspace_of_a_longer_prompt_serves_shorter_ones(fmt):
     assert chunk <= need[0]
 
 
+@pytest.mark.parametrize("fmt", [_lib.PE_WFMT_NF4, _lib.PE_WFMT_NF4_F32ABS, _lib.PE_WFMT_DENSE])
+@pytest.mark.parametrize("hidden,heads,kv_heads,intermediate", [
+    (512, 4, 2, 768), (512, 8, 8, 1408), (1024, 16, 8, 3072), (1024, 8, 2, 2816), (2048, 16, 16, 5632),
+    (4096, 32, 32, 11008)])
+def test_workspace_grows_with_every_row_at_every_width(fmt, hidden, heads, kv_heads, intermediate):
+    d = _desc_7b_nf4()
+    d.weight_format, d.hidden, d.num_heads, d.num_kv_heads = fmt, hidden, heads, kv_heads
+    d.intermediate = d.intermediate_padded = intermediate
+    need = [_lib.load().pe_forward_workspace_bytes(C.byref(d), m, 4096) for m in range(257, 2600)]
+    assert need[0] > 0 and all(b >= a for a, b in zip(need, need[1:]))
+
+
 @pytest.mark.parametrize("nbytes", [0, 4096, ops.ZEROED_BYTES, ops.ZEROED_BYTES + 1])
 def test_workspace_of_one_call(nbytes):
     calls = []
