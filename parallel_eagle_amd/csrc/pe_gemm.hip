@@ -1172,7 +1172,7 @@ __device__ __forceinline__ void t256_tile(uint8_t* smem, const T256Args& p, int 
     const int f = wave * PW + i;
     if (f < AF) {
       const int mt = min(mblock * p.bt + (f >> 1), p.mtiles - 1);
-      voff[i] = (uint32_t)(((mt * p.units * 8 + (f & 1)) * 64 + lane) * 16);
+      voff[i] = (uint32_t)((((int64_t)mt * p.units * 8 + (f & 1)) * 64 + lane) * 16);
     } else {
       const int nt = ntile * 8 + ((f - AF) >> 1);
       voff[i] = (uint32_t)((((int64_t)nt * p.units * 8 + 4 * g) * 64 + ln + 32 * (f & 1)) * 16);

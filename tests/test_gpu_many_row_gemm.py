@@ -33,3 +33,18 @@ def test_many_row_linear_matches_the_float64_product(dtype, m, n, k, pad):
     bound = half_ulp * ref.abs() * 1.01 + k * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T) + 2.0 ** -25
     assert bool(((out[:, :n].double() - ref).abs() <= bound).all())
     assert pad == 0 or bool((out[:, n:] == 7.0).all())
+
+
+def test_rows_past_two_gib():
+    """Byte offsets within X from 2 GiB on (up to 4 GiB the same kernel): the last rows of 2.2 GiB."""
+    m, n, k = 72001, 256, 16384
+    gen = torch.Generator(device=DEV).manual_seed(1)
+    x = torch.empty(m, k, dtype=torch.bfloat16, device=DEV).normal_(generator=gen)
+    w = (torch.randn(n, k, generator=gen, device=DEV) * 0.02).to(torch.bfloat16)
+    out = ops.linear(x, n, dense=ops.dense_repack(w))
+    rows = torch.cat([torch.arange(300, device=DEV), torch.arange(65400, 65700, device=DEV),
+                      torch.arange(m - 300, m, device=DEV)])
+    xr = x[rows].double()
+    ref = xr @ w.double().T
+    bound = 2.0 ** -8 * ref.abs() * 1.01 + k * 2.0 ** -24 * (xr.abs() @ w.double().abs().T)
+    assert bool(((out[rows].double() - ref).abs() <= bound).all())
