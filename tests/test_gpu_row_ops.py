@@ -29,9 +29,11 @@ def test_rmsnorm_rows(dtype, h, pad):
         assert bool(((got.double() - want.double()).abs() <= eps * want.double().abs() + floor).all())
 
 
-@pytest.mark.parametrize("m,k,ld,off", [(65, 128, 128, 0), (96, 384, 392, 0), (130, 256, 257, 0), (70, 512, 512, 1)])
+@pytest.mark.parametrize("m,k,ld,off", [(257, 128, 128, 0), (288, 384, 392, 0), (290, 256, 257, 0), (385, 512, 512, 1),
+                                        (513, 1152, 1160, 4), (300, 256, 256, 8)])
 def test_packing_of_many_rows(m, k, ld, off):
-    """pe_dense_gemm over more than 64 rows packs X: an identity weight returns X bit for bit."""
+    """pe_dense_gemm over more than 256 rows packs X (the last two columns: the
+    rows' stride and first element): an identity weight returns X bit for bit."""
     gen = torch.Generator(device=DEV).manual_seed(m)
     flat = torch.randn(m * ld + 8, generator=gen, device=DEV).to(torch.bfloat16)
     x = flat[off: off + m * ld].view(m, ld)[:, :k]
