@@ -1101,11 +1101,15 @@ __global__ __launch_bounds__(kWaves * 64, 2) void dense_gemm_bigm_kernel(const u
 // Dense 16-bit GEMM over many rows: 256 x 256 output tiles
 // ---------------------------------------------------------------------------
 // One workgroup = 4 waves = a block of up to 256 rows (32-row tiles of the
-// A-tiled X) x 256 columns (eight 32-column weight tiles); wave w owns the
-// row tiles MI (w / 2) .. + MI - 1 and the columns 128 (w % 2) .. + 127: MI x 4
-// MFMA tiles (MI = 4: 256 fp32 accumulators). A block of fewer tiles, the last
-// of a launch or all of a small one, runs MI = 3, 2 or 1 (777 rows: 3 x 256 +
-// 9, the 9 rows at the price of 64).
+// A-tiled X) x 256 columns (eight 32-column weight tiles). With an even count
+// 2 MI of row tiles, wave w owns the row tiles MI (w / 2) .. + MI - 1 and the
+// columns 128 (w % 2) .. + 127: MI x 4 MFMA tiles (MI = 4: 256 fp32
+// accumulators). With an odd count 2 MI - 1 (ODD) it owns all of them and the
+// columns 64 w .. + 63, so that the four waves share an odd block evenly: the
+// padded tile is staged but not multiplied (one fp16 layer and the 152064-column
+// lm_head over 150 and 200 rows: 619 and 696 us with it multiplied or on the
+// 128-column kernel, 591 and 657 like this). A block of fewer than eight tiles
+// is the last of a launch or all of a small one (777 rows: 3 x 256 + 9).
 //
 // K is walked in stages of two MFMA k-steps. A stage's 4 MI A fragments and 16
 // B fragments, 1 KiB each, go straight from global memory into an LDS ring of
@@ -1156,10 +1160,11 @@ struct T256Args {
   int vec;        // 16-bit output: rows and base 16-byte aligned
 };
 
-template <int DT, int MI, int EPI>
+template <int DT, int MI, bool ODD, int EPI>
 __device__ __forceinline__ void t256_tile(uint8_t* smem, const T256Args& p, int ntile, int mblock, int split, int u0,
                                           int nst) {
   constexpr int STG = t256_stage(MI), R = t256_ring(MI), PW = MI + 4, AF = 4 * MI;
+  constexpr int MW = ODD ? 2 * MI - 1 : MI, NW = ODD ? 2 : 4;  // this wave's row and column tiles
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int ln = lane & 31, g = lane >> 5;
   const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem;
@@ -1189,23 +1194,23 @@ __device__ __forceinline__ void t256_tile(uint8_t* smem, const T256Args& p, int 
       lds_dma16(wave * PW + i < AF ? (const void*)xs : (const void*)ws, voff[i],
                 __builtin_amdgcn_readfirstlane(dst + i * 1024));
   };
-  const int wm = wave >> 1, wn = wave & 1;
-  f32x16_t acc[MI][4];
+  const int wm = ODD ? 0 : wave >> 1, wn = ODD ? wave : wave & 1;
+  f32x16_t acc[MW][NW];
 #pragma unroll
-  for (int mi = 0; mi < MI; ++mi)
+  for (int mi = 0; mi < MW; ++mi)
 #pragma unroll
-    for (int ni = 0; ni < 4; ++ni)
+    for (int ni = 0; ni < NW; ++ni)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[mi][ni][r] = 0.f;
-  u32x4_t fa[2][MI], fb[2][4];
-  // fragment f (the four of B, then those of A) of k-step sl of the stage at `st`
+  u32x4_t fa[2][MW], fb[2][NW];
+  // fragment f (those of B, then those of A) of k-step sl of the stage at `st`
   auto read = [&](const uint8_t* st, int sl, int f) {
-    if (f < 4) fb[sl][f] = *(const u32x4_t*)(st + (AF + (4 * wn + f) * 2 + sl) * 1024 + lane * 16);
-    else fa[sl][f - 4] = *(const u32x4_t*)(st + ((MI * wm + f - 4) * 2 + sl) * 1024 + lane * 16);
+    if (f < NW) fb[sl][f] = *(const u32x4_t*)(st + (AF + (NW * wn + f) * 2 + sl) * 1024 + lane * 16);
+    else fa[sl][f - NW] = *(const u32x4_t*)(st + ((MI * wm + f - NW) * 2 + sl) * 1024 + lane * 16);
   };
   auto mul = [&](int sl, int mi) {
 #pragma unroll
-    for (int ni = 0; ni < 4; ++ni)
+    for (int ni = 0; ni < NW; ++ni)
       acc[mi][ni] = EPI == kEpiTF32 ? mfma16<DT>(fa[sl][mi], fb[sl][ni], acc[mi][ni])
                                     : mfma16<DT>(fb[sl][ni], fa[sl][mi], acc[mi][ni]);
   };
@@ -1214,7 +1219,7 @@ __device__ __forceinline__ void t256_tile(uint8_t* smem, const T256Args& p, int 
   __builtin_amdgcn_s_waitcnt(wait_vm_lgkm0((R - 2) * PW));
   lds_barrier();
 #pragma unroll
-  for (int f = 0; f < 4 + MI; ++f) read(smem, 0, f);
+  for (int f = 0; f < NW + MW; ++f) read(smem, 0, f);
   int slot = 0;  // of stage t
   for (int t = 0; t < nst; ++t) {
     const int next = slot + 1 == R ? 0 : slot + 1;
@@ -1223,11 +1228,11 @@ __device__ __forceinline__ void t256_tile(uint8_t* smem, const T256Args& p, int 
     const uint8_t* sn = smem + next * STG;
     // first k-step: the second one's fragments are read, stage t + R - 1 requested
 #pragma unroll
-    for (int mi = 0; mi < MI; ++mi) {
+    for (int mi = 0; mi < MW; ++mi) {
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int f = mi * (4 + MI) / MI; f < (mi + 1) * (4 + MI) / MI; ++f) read(st, 1, f);
-      issue(t + R - 1, free_slot, mi * PW / MI, (mi + 1) * PW / MI);
+      for (int f = mi * (NW + MW) / MW; f < (mi + 1) * (NW + MW) / MW; ++f) read(st, 1, f);
+      issue(t + R - 1, free_slot, mi * PW / MW, (mi + 1) * PW / MW);
       mul(0, mi);
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -1235,37 +1240,37 @@ __device__ __forceinline__ void t256_tile(uint8_t* smem, const T256Args& p, int 
     __builtin_amdgcn_s_waitcnt(wait_vm_lgkm0((R - 2) * PW));
     lds_barrier();
 #pragma unroll
-    for (int mi = 0; mi < MI; ++mi) {
+    for (int mi = 0; mi < MW; ++mi) {
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int f = mi * (4 + MI) / MI; f < (mi + 1) * (4 + MI) / MI; ++f) read(sn, 0, f);
+      for (int f = mi * (NW + MW) / MW; f < (mi + 1) * (NW + MW) / MW; ++f) read(sn, 0, f);
       mul(1, mi);
     }
     __builtin_amdgcn_sched_barrier(0);
     slot = next;
   }
   __builtin_amdgcn_s_waitcnt(0);  // the ring's last loads land before it is reused or the workgroup ends
-  const int row0 = mblock * p.bt * 32 + 32 * MI * wm, col0 = ntile * 256 + 128 * wn;
+  const int row0 = mblock * p.bt * 32 + 32 * MI * wm, col0 = ntile * 256 + 32 * NW * wn;
   if constexpr (EPI == kEpiTF32) {
     float* out = (float*)p.out + (int64_t)split * p.M * p.ld;
 #pragma unroll
-    for (int mi = 0; mi < MI; ++mi)
+    for (int mi = 0; mi < MW; ++mi)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int row = row0 + 32 * mi + 8 * (r >> 2) + 4 * g + (r & 3);
         if (row >= p.M) continue;
 #pragma unroll
-        for (int ni = 0; ni < 4; ++ni) out[(int64_t)row * p.ld + col0 + 32 * ni + ln] = acc[mi][ni][r];
+        for (int ni = 0; ni < NW; ++ni) out[(int64_t)row * p.ld + col0 + 32 * ni + ln] = acc[mi][ni][r];
       }
   } else if constexpr (EPI == kEpiTSwiglu) {
     typedef Elem<DT> E;
     // tiles 2 pr and 2 pr + 1 are the gate and up columns of 32 activation columns
 #pragma unroll
-    for (int mi = 0; mi < MI; ++mi) {
+    for (int mi = 0; mi < MW; ++mi) {
       const int row = row0 + 32 * mi + ln;
       if (row >= p.M) continue;
 #pragma unroll
-      for (int pr = 0; pr < 2; ++pr)
+      for (int pr = 0; pr < NW / 2; ++pr)
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           float o[4];
@@ -1280,15 +1285,16 @@ __device__ __forceinline__ void t256_tile(uint8_t* smem, const T256Args& p, int 
     }
   } else {
     __syncthreads();  // every wave is done with the ring: it becomes the output tile
-    uint8_t* mine = smem + wave * (MI * 32 * 256);
+    constexpr int CH = 4 * NW, PITCH = CH * 16;  // 16-byte chunks and bytes of a wave's row
+    uint8_t* mine = smem + wave * (MW * 32 * PITCH);
 #pragma unroll
-    for (int mi = 0; mi < MI; ++mi)
+    for (int mi = 0; mi < MW; ++mi)
 #pragma unroll
-      for (int ni = 0; ni < 4; ++ni)
+      for (int ni = 0; ni < NW; ++ni)
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           const int m = 32 * mi + ln, c = 4 * ni + q;
-          *(uint2*)(mine + m * 256 + ((c ^ (m & 15)) * 16) + 8 * g) =
+          *(uint2*)(mine + m * PITCH + ((c ^ (m & (CH - 1))) * 16) + 8 * g) =
               make_uint2(pack2_16<DT>(acc[mi][ni][4 * q], acc[mi][ni][4 * q + 1]),
                          pack2_16<DT>(acc[mi][ni][4 * q + 2], acc[mi][ni][4 * q + 3]));
         }
@@ -1296,9 +1302,9 @@ __device__ __forceinline__ void t256_tile(uint8_t* smem, const T256Args& p, int 
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
 #pragma unroll 4
-    for (int it = 0; it < MI * 8; ++it) {
-      const int m = it * 4 + (lane >> 4), c = lane & 15;
-      const u32x4_t v = *(const u32x4_t*)(mine + m * 256 + ((c ^ (m & 15)) * 16));
+    for (int it = 0; it < MW * CH / 2; ++it) {
+      const int m = it * (64 / CH) + lane / CH, c = lane & (CH - 1);
+      const u32x4_t v = *(const u32x4_t*)(mine + m * PITCH + ((c ^ (m & (CH - 1))) * 16));
       if (row0 + m >= p.M) continue;
       uint16_t* dst = (uint16_t*)p.out + (int64_t)(row0 + m) * p.ld + col0 + 8 * c;
       if (p.vec) {
@@ -1325,10 +1331,22 @@ __global__ __launch_bounds__(256, 1) void dense_gemm_t256_kernel(T256Args p) {
   const int u0 = split * p.ups, u1 = min(p.units, u0 + p.ups);
   if (u0 >= u1) return;
   const int left = min(p.bt, p.mtiles - mblock * p.bt);
-  if (left > 6) t256_tile<DT, 4, EPI>(smem, p, ntile, mblock, split, u0, (u1 - u0) * 4);
-  else if (left > 4) t256_tile<DT, 3, EPI>(smem, p, ntile, mblock, split, u0, (u1 - u0) * 4);
-  else if (left > 2) t256_tile<DT, 2, EPI>(smem, p, ntile, mblock, split, u0, (u1 - u0) * 4);
-  else t256_tile<DT, 1, EPI>(smem, p, ntile, mblock, split, u0, (u1 - u0) * 4);
+  const int nst = (u1 - u0) * 4;
+  // (the SwiGLU epilogue pads an odd count: with the odd forms beside the even
+  // ones its kernel spills accumulators in the loop)
+  constexpr bool kOdd = EPI != kEpiTSwiglu;
+  switch (left) {
+#define PE_T256_TILE(MI, ODD) t256_tile<DT, MI, ODD, EPI>(smem, p, ntile, mblock, split, u0, nst)
+    case 8: PE_T256_TILE(4, false); break;
+    case 7: PE_T256_TILE(4, kOdd); break;
+    case 6: PE_T256_TILE(3, false); break;
+    case 5: PE_T256_TILE(3, kOdd); break;
+    case 4: PE_T256_TILE(2, false); break;
+    case 3: PE_T256_TILE(2, kOdd); break;
+    case 2: PE_T256_TILE(1, false); break;
+    default: PE_T256_TILE(1, kOdd); break;
+#undef PE_T256_TILE
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -2146,13 +2164,10 @@ int pe_internal_dense_bigm(const void* x_tiled, int M, int K, const void* w, int
   // 256-column tiles from the LDS ring; the 128-column kernel keeps widths that
   // are not a multiple of 256 (M = 300, N = K = 4096: 39 against 72 us; 1500
   // rows, K = 11008: 176 against 203; the 152064-column lm_head over 70, 160
-  // and 777 rows 317, 356 and 1190 us against 352, 407 and 1742). Seven row
-  // tiles under a lm_head of more than a round of tiles stay there too: the
-  // padded eighth tile is an eighth more matrix-core work at full power, and in
-  // the batched pass (208 x 152064 x 5120, back to back) it cost 35 us (a lone
-  // launch: 411 against 433; 208 x 32000 x 4096, half a round: 70 against 87).
-  const bool padded = !f32_out && (M + 31) / 32 == 7 && N / 256 > cu_count();
-  if (t256_shape(M, N, K) && !padded) {
+  // and 777 rows 317, 356 and 1190 us against 352, 407 and 1742; a layer and
+  // that lm_head over 200 rows of a bf16 prompt 622 against 637, of an fp16 one
+  // 657 against 693, even (670 and 668) in a bf16 batch of 208 rows).
+  if (t256_shape(M, N, K)) {
     const T256Plan plan = t256_plan(M, N, K, splits && f32_out ? max_splits : 1, f32_out);
     if (splits) *splits = plan.S;
     return t256_launch(x_tiled, M, K, w, dtype, N, out, ld_out, f32_out ? kEpiTF32 : kEpiT16, 0, plan, st);

@@ -18,6 +18,9 @@ DEV = "cuda"
     (417, 768, 256, 0),     # five tiles and a ragged sixth
     (777, 256, 1152, 0),    # few column tiles: small row blocks
     (2047, 8192, 256, 0),   # full row blocks, one round of workgroups
+    (480, 65536, 128, 0),   # many column tiles, so large row blocks: a last one of seven tiles,
+    (410, 65536, 128, 1),   # of five, the last one ragged
+    (281, 65536, 128, 0),   # and of three
     (300, 384, 256, 0),     # N not a multiple of 256: the 128-column kernel
 ])
 def test_many_row_linear_matches_the_float64_product(dtype, m, n, k, pad):

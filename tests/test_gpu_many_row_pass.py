@@ -72,6 +72,22 @@ def test_causal_pass_at_once_equals_short_passes(target, rows, prefix):
     _close(caches[1].v[:, :, :n], caches[0].v[:, :, :n], target.dtype)
 
 
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
+def test_odd_row_blocks_of_the_fp32_partials(dtype):
+    """A wide q/k/v projection takes row blocks of up to eight 32-row tiles, the
+    last of 1, 3, 5 or 7."""
+    tm = _target(dtype, replace(SHAPE, num_layers=1, num_heads=96, num_kv_heads=48, feature_layers=(0, 1, 1)))
+    for rows in (145, 209, 321, 449):
+        ids = torch.randint(0, SHAPE.vocab, (rows,), generator=torch.Generator(device=DEV).manual_seed(rows), device=DEV)
+        pos = torch.arange(rows, device=DEV)
+        caches = [tm.make_cache(), tm.make_cache()]
+        want = [tm.forward_cached(ids[c: c + 64], caches[0], pos[c: c + 64])[0][0] for c in range(0, rows, 64)]
+        got = tm.forward_cached(ids, caches[1], pos)[0][0]
+        _close(got, torch.cat(want), tm.dtype)
+        for a, b in ((caches[1].k, caches[0].k), (caches[1].v, caches[0].v)):
+            _close(a[:, :, :rows], b[:, :, :rows], tm.dtype)
+
+
 @pytest.mark.parametrize("trees", [(40, 26), (64, 64, 30, 7), (60,) * 5])
 def test_batched_pass_equals_its_sequences_alone(target, trees):
     gen = torch.Generator(device=DEV).manual_seed(sum(trees))
