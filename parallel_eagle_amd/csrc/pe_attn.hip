@@ -2191,6 +2191,12 @@ extern "C" int64_t pe_attention_workspace_bytes(int T, int nh, int nkv, int hd, 
   return attention_workspace_bytes(T, nh, nkv, hd, kv_len, dtype, PE_ATTN_SDPA);
 }
 
+// Row blocks for eager attention from the row count of attn_rows_kernel on,
+// though at 256 rows they launch fewer workgroups than one-tile attention (64
+// against 256 at 32 heads): a draft of one layer, one-tile time over row-block
+// time, 1.00 at 260 to 300 rows, 0.99 to 1.00 at 350 to 450, 1.02 at 520 and
+// 1.06 at 1500 (32 / 32 heads); 1.00 to 1.01 at 260 to 450, 1.01 at 520 and 1.07
+// at 1500 (40 / 8 heads); 0.99 at 160 to 250 in both.
 bool pe_internal_eager_tiles(int T, int mask_mode) { return mask_mode == PE_MASK_CAUSAL && T >= kRowsMinNodes; }
 
 int pe_internal_tree_attention(const void* q, const void* k_cache, const void* v_cache, int64_t cache_cap, int nh,
