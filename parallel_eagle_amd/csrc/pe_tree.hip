@@ -131,7 +131,7 @@ constexpr int kArgThreads = 1024;
 // conversion, a NaN test and a 32-bit key per element; the best vector is kept
 // whole and searched once at the end. NaNs (a magnitude past infinity's) are
 // only detected: `nan` then tells the caller that the result counts numbers
-// only. kArgVec vectors (a 152064-element row's whole share) are in flight at
+// only (fp32 keys hold them). kArgVec vectors (a 152064-element row's whole share) are in flight at
 // a time; one workgroup reads a row, so its CU's load rate is the bound
 // (26 rows of 152064 bf16 elements: 18.5 us with 32-bit keys and 8 vectors in
 // flight, 12.8 us like this).
@@ -160,9 +160,7 @@ __device__ __forceinline__ void share_best(const typename Elem<DT>::T* __restric
         if (vi < nvec) {
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
-            const float v = __uint_as_float(buf[k][j]);
-            nan |= v != v;
-            const uint32_t key = arg_key(v);
+            const uint32_t key = arg_key(__uint_as_float(buf[k][j]));
             if (key > bk) {
               bk = key;
               bi = (int)(vi * kPer + j);
@@ -227,13 +225,14 @@ __device__ __forceinline__ void share_best(const typename Elem<DT>::T* __restric
   }
   for (int64_t i = nvec * kPer + threadIdx.x; i < V; i += kArgThreads) {
     const float v = Elem<DT>::load(x, i);
-    nan |= v != v;
+    if constexpr (DT != PE_DTYPE_F32) nan |= v != v;
     const uint32_t key = arg_key(v);
     if (key > bk) {
       bk = key;
       bi = (int)i;
     }
   }
+  if constexpr (DT == PE_DTYPE_F32) nan = bk == 0xFFFFFFFFu;  // a NaN's key, the largest
 }
 
 // Whole 16-byte vectors of a row (none when it is not 16-byte aligned).
@@ -243,23 +242,29 @@ __device__ __forceinline__ int64_t row_vectors(const typename Elem<DT>::T* x, in
 }
 
 // One block of kArgThreads per row: every thread's best, then the block's with
-// (key descending, index ascending). A row with a NaN is searched again for
-// its first NaN (every NaN has the largest key).
+// (key descending, index ascending). A thread whose 16-bit share holds a NaN
+// goes through its vectors again for the first one (every NaN has the largest
+// key); the fp32 search and the single elements have its key already.
 template <int DT>
 __device__ int row_argmax(const typename Elem<DT>::T* __restrict__ x, int64_t V, int32_t* out) {
   uint32_t bk;
   int bi;
   bool nan;
-  share_best<DT>(x, V, row_vectors<DT>(x, V), bk, bi, nan);
-  if (__syncthreads_or(nan)) {
-    bk = 0;
-    bi = -1;
-    for (int64_t i = threadIdx.x; i < V; i += kArgThreads) {
-      const uint32_t key = arg_key(Elem<DT>::load(x, i));
-      if (key > bk) {
-        bk = key;
-        bi = (int)i;
-      }
+  const int64_t nvec = row_vectors<DT>(x, V);
+  share_best<DT>(x, V, nvec, bk, bi, nan);
+  if constexpr (DT != PE_DTYPE_F32) {
+    if (nan) {
+      constexpr int kPer = 8;
+      bool found = false;
+      for (int64_t vi = threadIdx.x; vi < nvec && !found; vi += kArgThreads)
+        for (int j = 0; j < kPer && !found; ++j) {
+          const float v = Elem<DT>::load(x, vi * kPer + j);
+          if (v != v) {
+            bk = arg_key(v);
+            bi = (int)(vi * kPer + j);
+            found = true;
+          }
+        }
     }
   }
   auto better = [](uint32_t k2, int i2, uint32_t k1, int i1) {  // (k2, i2) beats (k1, i1)
