@@ -1105,10 +1105,11 @@ __global__ __launch_bounds__(kWaves * 64, 2) void dense_gemm_bigm_kernel(const u
 // 2 MI of row tiles, wave w owns the row tiles MI (w / 2) .. + MI - 1 and the
 // columns 128 (w % 2) .. + 127: MI x 4 MFMA tiles (MI = 4: 256 fp32
 // accumulators). With an odd count 2 MI - 1 (ODD) it owns all of them and the
-// columns 64 w .. + 63, so that the four waves share an odd block evenly: the
-// padded tile is staged but not multiplied (one fp16 layer and the 152064-column
-// lm_head over 150 and 200 rows: 619 and 696 us with it multiplied or on the
-// 128-column kernel, 591 and 657 like this). A block of fewer than eight tiles
+// columns 64 w .. + 63, so that the four waves share an odd block evenly and the
+// tile that pads it is neither staged nor multiplied (one fp16 layer and the
+// 152064-column lm_head over 150 and 200 rows: 606 and 692 us with it multiplied
+// or on the 128-column kernel, 584 and 641 like this; 598 and 644 with it staged
+// only). A block of fewer than eight tiles
 // is the last of a launch or all of a small one (777 rows: 3 x 256 + 9).
 //
 // K is walked in stages of two MFMA k-steps. A stage's 4 MI A fragments and 16
@@ -1164,6 +1165,8 @@ template <int DT, int MI, bool ODD, int EPI>
 __device__ __forceinline__ void t256_tile(uint8_t* smem, const T256Args& p, int ntile, int mblock, int split, int u0,
                                           int nst) {
   constexpr int STG = t256_stage(MI), R = t256_ring(MI), PW = MI + 4, AF = 4 * MI;
+  constexpr int kPadWave = (AF - 2) / PW;  // ODD: the wave whose two fragments of the last row tile are left out
+  static_assert((AF - 1) / PW == kPadWave, "one wave owns the padded tile's fragments");
   constexpr int MW = ODD ? 2 * MI - 1 : MI, NW = ODD ? 2 : 4;  // this wave's row and column tiles
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int ln = lane & 31, g = lane >> 5;
@@ -1190,9 +1193,16 @@ __device__ __forceinline__ void t256_tile(uint8_t* smem, const T256Args& p, int 
     const uint8_t* ws = wb + (int64_t)(8 * (tt >> 2) + (tt & 3)) * 1024;
     const uint32_t dst = lds_base + slot * STG + wave * (PW * 1024);
 #pragma unroll
-    for (int i = i0; i < i1; ++i)
+    for (int i = i0; i < i1; ++i) {
+      if (ODD && wave == kPadWave && (wave * PW + i == AF - 2 || wave * PW + i == AF - 1)) continue;
       lds_dma16(wave * PW + i < AF ? (const void*)xs : (const void*)ws, voff[i],
                 __builtin_amdgcn_readfirstlane(dst + i * 1024));
+    }
+  };
+  // this wave's fragments are in registers, and its loads up to the stage before the last R - 2 requested have landed
+  auto landed = [&]() {
+    if (ODD && wave == kPadWave) __builtin_amdgcn_s_waitcnt(wait_vm_lgkm0((R - 2) * (PW - 2)));
+    else __builtin_amdgcn_s_waitcnt(wait_vm_lgkm0((R - 2) * PW));
   };
   const int wm = ODD ? 0 : wave >> 1, wn = ODD ? wave : wave & 1;
   f32x16_t acc[MW][NW];
@@ -1216,7 +1226,7 @@ __device__ __forceinline__ void t256_tile(uint8_t* smem, const T256Args& p, int 
   };
 #pragma unroll
   for (int t = 0; t < R - 1; ++t) issue(t, t, 0, PW);
-  __builtin_amdgcn_s_waitcnt(wait_vm_lgkm0((R - 2) * PW));
+  landed();
   lds_barrier();
 #pragma unroll
   for (int f = 0; f < NW + MW; ++f) read(smem, 0, f);
@@ -1237,7 +1247,7 @@ __device__ __forceinline__ void t256_tile(uint8_t* smem, const T256Args& p, int 
     }
     __builtin_amdgcn_sched_barrier(0);
     // this wave has its last fragments of stage t, and its loads of stage t + 1 have landed
-    __builtin_amdgcn_s_waitcnt(wait_vm_lgkm0((R - 2) * PW));
+    landed();
     lds_barrier();
 #pragma unroll
     for (int mi = 0; mi < MW; ++mi) {
@@ -2165,8 +2175,8 @@ int pe_internal_dense_bigm(const void* x_tiled, int M, int K, const void* w, int
   // are not a multiple of 256 (M = 300, N = K = 4096: 39 against 72 us; 1500
   // rows, K = 11008: 176 against 203; the 152064-column lm_head over 70, 160
   // and 777 rows 317, 356 and 1190 us against 352, 407 and 1742; a layer and
-  // that lm_head over 200 rows of a bf16 prompt 622 against 637, of an fp16 one
-  // 657 against 693, even (670 and 668) in a bf16 batch of 208 rows).
+  // that lm_head over 200 rows of a bf16 prompt 612 against 632, of an fp16 one
+  // 641 against 692, in a bf16 batch of 208 rows 655 against 662).
   if (t256_shape(M, N, K)) {
     const T256Plan plan = t256_plan(M, N, K, splits && f32_out ? max_splits : 1, f32_out);
     if (splits) *splits = plan.S;
